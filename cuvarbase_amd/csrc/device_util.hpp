@@ -96,15 +96,40 @@ __device__ __forceinline__ int spread_exponent(float bound) {
     return e < -120 ? -120 : (e > 120 ? 120 : e);
 }
 
-// exp(2 pi i r) for a phase r given in revolutions as FP64: the integer part
-// is removed in FP64 (r - rint(r) in [-1/2, 1/2]) and only the reduced phase
-// is evaluated in FP32.
-__device__ __forceinline__ float2 expi_rev(double r) {
-    const float rr = (float)(r - rint(r));
-    float s, c;
-    sincospif(2.0f * rr, &s, &c);
-    return make_float2(c, s);
+// cos and sin of (pi/2) (x + quarter), |x| <= 1/2: minimax polynomials in x^2
+// fitted to the absolute error over that range (pi/2 in two parts, so that the
+// sine is off by half an ulp, 4.2e-8, and the cosine by one, 5.8e-8, in FP32
+// arithmetic), then the quarter turns by exchange and sign
+__device__ __forceinline__ float2 expi_quarter(float x, uint32_t quarter) {
+    const float u = x * x;
+    float ps = fmaf(u, -4.600198474e-03f, 7.967966795e-02f);
+    ps = fmaf(u, ps, -6.459634900e-01f);
+    ps = fmaf(u, ps, -4.371138829e-08f);
+    const float s = fmaf(x, 1.570796371e+00f, x * ps);
+    float pc = fmaf(u, 9.040216682e-04f, -2.086028829e-02f);
+    pc = fmaf(u, pc, 2.536692321e-01f);
+    pc = fmaf(u, pc, -1.233700514e+00f);
+    const float c = fmaf(u, pc, 1.0f);
+    const bool odd = (quarter & 1u) != 0u;
+    const float cs = odd ? s : c, sn = odd ? c : s;
+    // cosine changes sign in quarters 1 and 2, sine in 2 and 3
+    return make_float2(__uint_as_float(__float_as_uint(cs) ^ (((quarter + 1u) & 2u) << 30)),
+                       __uint_as_float(__float_as_uint(sn) ^ ((quarter & 2u) << 30)));
 }
+
+// exp(2 pi i y / 4) for a phase y in quarter turns as FP64: adding 1.5 2^52
+// rounds y to whole quarters (|y| < 2^51), the low word of the sum is their
+// count modulo 2^32, and only the rest, at most 1/2, is rounded to FP32.  A
+// phase that is not finite gives NaN.
+__device__ __forceinline__ float2 expi_turn4(double y) {
+    constexpr double kRound = 6755399441055744.0;   // 1.5 2^52
+    const double t = y + kRound;
+    const float x = (float)(y - (t - kRound));
+    return expi_quarter(x, (uint32_t)__double2loint(t));
+}
+
+// exp(2 pi i r) for a phase r given in revolutions as FP64
+__device__ __forceinline__ float2 expi_rev(double r) { return expi_turn4(4.0 * r); }
 
 // Buffer access to one curve's grid region (at most 3 grids of 2^24
 // complex64 cells, under 2^32 bytes): the base address and size live in a

@@ -230,9 +230,15 @@ hipError_t launch_pass2_lomb(int p2, int cr, int n1, const CurveGeom* bgeom,
 hipError_t launch_pass2_nfft(int p2, int cr, int n1, const CurveGeom* bgeom,
                              const CurveState* state, int ncurves, const float2* grids,
                              const PlanParams& pp, float2* out, hipStream_t s);
+// direct sums: workgroups of kDirNT threads, one per tile; a wave takes
+// kDirTile consecutive frequencies of a linear grid, or 64 of a frequency
+// list, and ws waves (1, 2, 4 or 8) share them, so that a tile has 8 / ws times
+// as many
+constexpr int kDirNT = 512;
+constexpr int kDirTile = 512;
 hipError_t launch_dirsum(const CurveGeom* d_geom, const CurveState* state,
                          const int32_t* tile_curve, const int32_t* tile_first,
-                         int ntiles, int rf, PointArrays pa,
+                         int ntiles, int ws, PointArrays pa,
                          const PlanParams& pp, void* power, int out_f64,
                          hipStream_t s);
 // direct FP64 sums for a curve's lowest frequencies, f_k (t_max - t_min) <
@@ -245,7 +251,7 @@ hipError_t launch_lowfreq(const CurveGeom* d_geom, const int32_t* small, int nsm
                           WideAux* aux, hipStream_t s);
 hipError_t launch_dirsum_custom(const CurveGeom* d_geom, const CurveState* state,
                                 const int32_t* tile_curve, const int32_t* tile_first,
-                                int ntiles, PointArrays pa, const PlanParams& pp,
+                                int ntiles, int ws, PointArrays pa, const PlanParams& pp,
                                 const double* freqs, void* power, int out_f64,
                                 hipStream_t s);
 hipError_t launch_gaussian_grid(const double* t, const double* y, int n_obs,

@@ -52,7 +52,7 @@ struct gls_plan {
     std::vector<int32_t> bcurves;  // curve indices of the entries, in order
     int64_t chunk_bytes = 0;       // > 0: grid region reused by every entry
     int ntiles = 0;         // direct method
-    int rf = 1;
+    int dir_ws = 8;         // waves per direct-sum tile
     // host image of the descriptors uploaded into workspace[0 .. meta.size())
     std::vector<char> meta;
     size_t off_geom = 0, off_bgeom = 0, off_tiles = 0, off_prep = 0;
@@ -127,6 +127,8 @@ std::atomic<int64_t> g_max_launch_items{kMaxLaunchItems};
 std::mutex g_tile_mu;
 std::map<std::pair<int, int>, BucketTiles> g_tile_override;   // gls_tile_set
 std::map<std::pair<int, int>, double> g_cost_override;        // gls_grid_cost_set
+
+constexpr int kWaveFreqs = 64;   // frequencies of a list per wave of direct sums
 
 constexpr int kNumRowSizes = kMaxLog2Row - kMinLog2Row + 1;
 
@@ -408,25 +410,40 @@ int plan_nfft_geometry(gls_plan* P, int ngrids, Layout& L, int64_t total_pts,
 }
 
 int plan_direct_tiles(gls_plan* P, std::vector<int32_t>& tiles) {
-    int rf = (P->pp.method == GLS_METHOD_DIRECT_CUSTOM) ? 1 : 8;
-    while (rf > 1) {
+    const bool custom = P->pp.method == GLS_METHOD_DIRECT_CUSTOM;
+    auto count = [&](int64_t per) {
         int64_t nt = 0;
-        for (auto& G : P->geom) nt += (G.nf + 256 * rf - 1) / (256 * rf);
-        if (nt >= 512) break;
-        rf >>= 1;
-    }
-    std::vector<int32_t> tc, tf;
-    for (int i = 0; i < P->ncurves; ++i) {
-        const int nf = P->geom[i].nf;
-        for (int k = 0; k < nf; k += 256 * rf) {
-            tc.push_back(i);
-            tf.push_back(k);
-        }
-    }
-    // one launch of 256-thread workgroups, one per tile
-    if ((int64_t)tc.size() * 256 > kMaxLaunchItems)
+        for (auto& G : P->geom) nt += (G.nf + per - 1) / per;
+        return nt;
+    };
+    // (2^23 tiles of 2,048 frequencies, 256 for lists: what one plan may hold)
+    if (count(custom ? 256 : 2048) > kMaxLaunchItems / 256)
         return fail(GLS_E_UNSUPPORTED, "too many direct-sum tiles for one launch: split the batch");
-    P->rf = rf;
+    // waves per tile: as few as still leave kDirTiles workgroups (two per
+    // compute unit) with at most a quarter of the waves without frequencies,
+    // and never so many that a wave has under kDirPoints points (waves that
+    // share a tile pay for adding their sums up: with 30-80 points per curve,
+    // 8 waves took 3 us longer than one)
+    constexpr int kDirTiles = 512, kDirPoints = 32;
+    const int64_t wave = custom ? kWaveFreqs : kDirTile;
+    const int64_t waves = count(wave);
+    int64_t pts = 0;   // points over all waves' frequencies
+    for (auto& G : P->geom) pts += (G.nf + wave - 1) / wave * G.n_obs;
+    int ws = 1;
+    while (ws < 8) {
+        const int64_t nt = count(wave * (8 / ws));
+        if (nt >= kDirTiles && 4 * waves >= 3 * nt * (8 / ws)) break;
+        if (pts < 2 * ws * kDirPoints * waves) break;
+        ws *= 2;
+    }
+    const int64_t per = wave * (8 / ws);
+    std::vector<int32_t> tc, tf;
+    for (int i = 0; i < P->ncurves; ++i)
+        for (int64_t k = 0; k < P->geom[i].nf; k += per) {
+            tc.push_back(i);
+            tf.push_back((int32_t)k);
+        }
+    P->dir_ws = ws;
     P->ntiles = (int)tc.size();
     tiles = tc;
     tiles.insert(tiles.end(), tf.begin(), tf.end());
@@ -575,7 +592,8 @@ void reserve_meta(gls_plan* P, Layout& L, size_t nbcurves, size_t ntiles_ints) {
 
 void fill_meta(gls_plan* P, const std::vector<int32_t>& bcurves,
                const std::vector<int32_t>& tiles) {
-    P->meta.assign(P->off_tiles + sizeof(int32_t) * tiles.size(), 0);
+    // (whole 16-byte words: the upload is then one launch)
+    P->meta.assign(align_up(P->off_tiles + sizeof(int32_t) * tiles.size(), 16), 0);
     if (!P->prep_list.empty())
         std::memcpy(P->meta.data() + P->off_prep, P->prep_list.data(),
                     sizeof(int32_t) * P->prep_list.size());
@@ -703,11 +721,11 @@ int run_plan(gls_plan* P, const double* t, const void* a, const void* b, void* o
         }
     } else if (P->pp.method == GLS_METHOD_DIRECT_CUSTOM) {
         GLS_HIP_TRY(launch_dirsum_custom(d_geom, state, d_tiles, d_tiles + P->ntiles, P->ntiles,
-                                         pa, P->pp, freqs, out, out_f64, s));
+                                         P->dir_ws, pa, P->pp, freqs, out, out_f64, s));
         GLS_HIP_TRY(mark());
     } else {
-        GLS_HIP_TRY(launch_dirsum(d_geom, state, d_tiles, d_tiles + P->ntiles, P->ntiles, P->rf,
-                                  pa, P->pp, out, out_f64, s));
+        GLS_HIP_TRY(launch_dirsum(d_geom, state, d_tiles, d_tiles + P->ntiles, P->ntiles,
+                                  P->dir_ws, pa, P->pp, out, out_f64, s));
         GLS_HIP_TRY(mark());
     }
     return GLS_OK;
