@@ -85,6 +85,22 @@ __device__ __forceinline__ T block_max(T v, T* scratch) {
     return r;
 }
 
+// Hand a value to other workgroups of the launch: an agent-scope exchange whose
+// result is waited for, so it has taken effect at the device's coherence point
+// when the call returns (a counter increased afterwards then announces it),
+// and agent-scope loads to read it.  A __threadfence would do the same by
+// writing back every dirty line of the die's L2, tens of microseconds after a
+// kernel that wrote much.
+__device__ __forceinline__ void agent_publish(double* p, double v) {
+    const unsigned long long old =
+        __hip_atomic_exchange((unsigned long long*)p, (unsigned long long)__double_as_longlong(v),
+                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("" ::"v"(old));
+}
+__device__ __forceinline__ double agent_load(const double* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Exponent e of the fixed-point spreading scale 2^e of an LDS tile whose
 // cells can hold at most `bound` in magnitude: scaled cells stay below 2^30,
 // half the int32 range.  Clamped to the FP32 exponent range.
@@ -126,6 +142,36 @@ __device__ __forceinline__ float2 expi_turn4(double y) {
     const double t = y + kRound;
     const float x = (float)(y - (t - kRound));
     return expi_quarter(x, (uint32_t)__double2loint(t));
+}
+
+// the same in FP64 throughout: Taylor polynomials of sine and cosine up to
+// x^15 and x^16, whose next terms are below 1e-17 at |x| = 1/2
+__device__ __forceinline__ double2 expi64_turn4(double y) {
+    constexpr double kRound = 6755399441055744.0;   // 1.5 2^52
+    constexpr double h = 1.57079632679489661923;    // pi/2
+    constexpr double h2 = h * h, h4 = h2 * h2, h6 = h4 * h2, h8 = h4 * h4;
+    const double t = y + kRound;
+    const double x = y - (t - kRound);
+    const uint32_t q = (uint32_t)__double2loint(t);
+    const double u = x * x;
+    double ps = fma(u, -h * h6 * h8 / 1307674368000.0, h * h4 * h8 / 6227020800.0);
+    ps = fma(u, ps, -h * h2 * h8 / 39916800.0);
+    ps = fma(u, ps, h * h8 / 362880.0);
+    ps = fma(u, ps, -h * h6 / 5040.0);
+    ps = fma(u, ps, h * h4 / 120.0);
+    ps = fma(u, ps, -h * h2 / 6.0);
+    ps = fma(u, ps, h);
+    double pc = fma(u, h8 * h8 / 20922789888000.0, -h6 * h8 / 87178291200.0);
+    pc = fma(u, pc, h4 * h8 / 479001600.0);
+    pc = fma(u, pc, -h2 * h8 / 3628800.0);
+    pc = fma(u, pc, h8 / 40320.0);
+    pc = fma(u, pc, -h6 / 720.0);
+    pc = fma(u, pc, h4 / 24.0);
+    pc = fma(u, pc, -h2 / 2.0);
+    const double s = x * ps, c = fma(u, pc, 1.0);
+    const bool odd = (q & 1u) != 0u;
+    const double cs = odd ? s : c, sn = odd ? c : s;
+    return make_double2((q + 1u) & 2u ? -cs : cs, q & 2u ? -sn : sn);
 }
 
 // exp(2 pi i r) for a phase r given in revolutions as FP64

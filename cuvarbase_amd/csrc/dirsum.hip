@@ -21,8 +21,6 @@ namespace gls {
 
 namespace {
 
-constexpr int NT = 256;
-
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 // points of one wave between two folds of its FP32 sums into FP64
@@ -249,205 +247,251 @@ __global__ __launch_bounds__(kDirNT) void dirsum_custom_kernel(
 // The GLS is ill-conditioned where a frequency spans few cycles over the
 // baseline (CC SS - CS^2 -> 0): there the FP32 round-off of the NFFT sums,
 // largest at the band edge where the lowest frequencies sit, reaches |dP| ~
-// 1e-4.  These few frequencies are recomputed by direct sums with FP64
-// phases and FP64 accumulation.
-// Grid (curve, group of 4 frequencies), the groups strided over the
-// frequencies from kbegin on: each wave of a block takes one frequency and
-// its 64 lanes stride over the curve's points (FP64 phases, FP64 sums), then
-// reduce by shuffles.  A block stops at the first group past the curve's low
-// frequencies, so however many there are (fine grids have hundreds), every
-// one is covered.
-constexpr int kLowPerBlock = NT / kWave;
-constexpr int kLowGroups = kLowMax / kLowPerBlock;   // blocks per curve
+// 1e-4.  These few frequencies, the leading run of the grid with |f| (t_max -
+// t_min) < kLowCycles, are recomputed by direct sums with FP64 phases and FP64
+// accumulation.
+//
+// A workgroup sums kLowGroup consecutive frequencies over a curve's points, or
+// over one of S slices of them: a point's phasor at the group's first frequency
+// and the phasor of one grid step are evaluated in FP64, the group's other
+// frequencies follow by FP64 products (kLowGroup - 1 of them, 1e-16 each).
+// Groups and slices are tasks that the curve's workgroups take in turn, so
+// however long the run is, every frequency is covered, and the sums of a curve
+// do not depend on how many workgroups it got.  Bound by FP64 issue: about 30
+// vector instructions per point and frequency (110 with a sine and cosine of
+// its own for each) and, for few points, by the chain of loads, exchanges and
+// the power.  Measured, against a sine and cosine per point and frequency, one
+// wave per frequency (1,024 lanes x 8 workgroups for wide curves) and two
+// launches: 2,000 curves of 20-300 points 64 -> 31 us, one of 1,000 points 15
+// -> 6 us, 37 of 400-3,000 points 28 -> 12 us, 32 of 100-50,000 points 89 -> 28
+// us, one of 200,000 points 32 -> 17 us.
+constexpr int kLowNT = 256;
+constexpr int kLowSums = 6 * kLowGroup;
+constexpr int kLowShort = 256;   // points up to which a wave sums alone
 
-// the six FP64 sums of frequency k over the curve's points and its power
-template <int OUT, bool WIDE, int BT, int LANES>
-__device__ __forceinline__ void lowfreq_one(const CurveGeom& G, const CurveState& st,
-                                            const PointArrays& pa, const PlanParams& pp, int k,
-                                            int tid, int lane, int N, double (*red)[6],
-                                            void* __restrict__ out) {
-    const double f = G.f0 + (double)k * G.df;
-    double acc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int j = lane; j < N; j += LANES) {
-        const double x = f * pa.dt[G.pts + j];
-        double sn, cs;
-        sincospi(2.0 * (x - rint(x)), &sn, &cs);
-        const double w = pa.w[G.pts + j], yw = pa.yw[G.pts + j];
-        acc[0] += w * cs;
-        acc[1] += w * sn;
-        acc[2] += w * (cs * cs - sn * sn);
-        acc[3] += w * (2.0 * cs * sn);
-        acc[4] += yw * cs;
-        acc[5] += yw * sn;
-    }
+// number of leading low frequencies of a curve
+__device__ __forceinline__ int low_count(const CurveGeom& G, double tspan) {
+    auto low = [&](int k) { return fabs(G.f0 + (double)k * G.df) * tspan < kLowCycles; };
+    if (!low(0)) return 0;
+    // the run ends near (kLowCycles / tspan - f0) / df, exactly where low() says
+    const double e = (kLowCycles / tspan - G.f0) / G.df;
+    int k = e < (double)G.nf ? max(1, (int)e) : G.nf;
+    while (k < G.nf && low(k)) ++k;
+    while (k > 1 && !low(k - 1)) --k;
+    return k;
+}
+
+// sums V values over lanes that differ in the bits HI, HI / 2 .. 1 of their
+// number: an exchange per value, but each step halves the values a lane holds
+// while their number is even.  Afterwards v[0 .. V/8) of a lane are the sums
+// number first .. (the same in lanes that differ in the remaining bits);
+// returns first
+template <int V, int HI>
+__device__ __forceinline__ int lane_sum_scatter(double (&v)[V], int lane) {
+    static_assert(V % 8 == 0 && V % 16 != 0 && HI >= 4, "three halvings");
+    int first = 0;
+    int cnt = V;
 #pragma unroll
-    for (int q = 0; q < 6; ++q) acc[q] = wave_sum(acc[q]);
-    if (WIDE) {
-        const int wv = tid / kWave;
-        if ((tid & (kWave - 1)) == 0)
-            for (int q = 0; q < 6; ++q) red[wv][q] = acc[q];
-        __syncthreads();
-        if (tid == 0)
-            for (int w = 1; w < BT / kWave; ++w)
-                for (int q = 0; q < 6; ++q) acc[q] += red[w][q];
-        __syncthreads();   // red is reused by the block's next frequency
+    for (int o = HI; o >= 1; o >>= 1) {
+        if (cnt % 2 == 0) {
+            cnt /= 2;
+            const bool up = (lane & o) != 0;
+            first += up ? cnt : 0;
+#pragma unroll
+            for (int i = 0; i < cnt; ++i) {
+                const double send = up ? v[i] : v[cnt + i];
+                const double keep = up ? v[cnt + i] : v[i];
+                v[i] = keep + __shfl_xor(send, o, kWave);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < cnt; ++i) v[i] += __shfl_xor(v[i], o, kWave);
+        }
     }
-    if (lane == 0) {
-        const double P = gls_power(acc[0], acc[1], acc[2], acc[3], acc[4], acc[5], st.yy,
-                                   st.ybar, pp.mode, pp.reg_c, pp.reg_s);
+    return first;
+}
+
+// adds the points j0, j0 + step .. below j1 of a curve to the sums of the
+// kLowGroup frequencies from k0 on
+__device__ __forceinline__ void low_points(const CurveGeom& G, const PointArrays& pa, int k0,
+                                           int j0, int j1, int step, double (&acc)[kLowSums]) {
+    const double f4 = 4.0 * (G.f0 + (double)k0 * G.df), df4 = 4.0 * G.df;
+    const double* const dt = pa.dt + G.pts;
+    const float* const pw = pa.w + G.pts;
+    const float* const py = pa.yw + G.pts;
+    double xn = 0.0;
+    float wn = 0.f, yn = 0.f;
+    if (j0 < j1) {
+        xn = dt[j0];
+        wn = pw[j0];
+        yn = py[j0];
+    }
+    for (int j = j0; j < j1; j += step) {
+        const double x = xn, w = wn, yw = yn;
+        if (j + step < j1) {   // the next point, loaded ahead
+            xn = dt[j + step];
+            wn = pw[j + step];
+            yn = py[j + step];
+        }
+        double2 e = expi64_turn4(f4 * x);
+        const double2 r = expi64_turn4(df4 * x);
+#pragma unroll
+        for (int i = 0; i < kLowGroup; ++i) {
+            double* a = acc + 6 * i;
+            a[0] += w * e.x;
+            a[1] += w * e.y;
+            a[2] += w * (e.x * e.x - e.y * e.y);
+            a[3] += w * (2.0 * e.x * e.y);
+            a[4] += yw * e.x;
+            a[5] += yw * e.y;
+            e = make_double2(e.x * r.x - e.y * r.y, e.x * r.y + e.y * r.x);
+        }
+    }
+}
+
+// Workgroups: bs for each of the nsmall curves of the list, then bw for each of
+// the wide ones after them (those with a record in aux may split their points).
+template <int OUT>
+__global__ __launch_bounds__(kLowNT) void lowfreq_kernel(
+    const CurveGeom* __restrict__ geom, const int32_t* __restrict__ list, int nsmall, int bs,
+    int bw, const CurveState* __restrict__ state, PointArrays pa, PlanParams pp,
+    WideAux* __restrict__ aux, void* __restrict__ out) {
+    constexpr int WAVES = kLowNT / kWave;
+    __shared__ double red[WAVES][4][kLowSums];
+    __shared__ int last;
+    const int tid = threadIdx.x;
+    const int lane = tid & (kWave - 1);
+    const int wv = tid / kWave;
+    const int bid = blockIdx.x;
+    const bool wide = bid >= nsmall * bs;
+    const int wi = wide ? (bid - nsmall * bs) / bw : 0;   // which of the wide curves
+    const int c = list[wide ? nsmall + wi : bid / bs];
+    const int first_task = wide ? (bid - nsmall * bs) % bw : bid % bs;
+    const int nblocks = wide ? bw : bs;
+    const CurveGeom& G = geom[c];
+    const CurveState st = state[c];
+    const int kl = G.n_obs > 0 ? low_count(G, st.tspan) : 0;
+    const int ngroups = (kl + kLowGroup - 1) / kLowGroup;
+    const int N = G.n_obs;
+    auto store = [&](int k, const double* a) {
+        const double P = gls_power(a[0], a[1], a[2], a[3], a[4], a[5], st.yy, st.ybar, pp.mode,
+                                   pp.reg_c, pp.reg_s);
         if (OUT == 0) ((float*)out)[G.out + k] = (float)P;
         else ((double*)out)[G.out + k] = P;
-    }
-}
-
-// WIDE: one frequency per 1024-thread block, all its lanes over the points
-// (long curves: 16 waves per frequency hide the FP64 latency).
-constexpr int kLowWideNT = 1024;
-// LOOP: the block strides on over the grid (gridDim.y groups apart) until it
-// passes the curve's low run; without it, one group per block (fewer live
-// registers: the common case, launched with enough groups for kLowMax
-// frequencies, and LOOP launches take any frequencies after those)
-template <int OUT, bool WIDE, bool LOOP>
-__global__ __launch_bounds__(WIDE ? kLowWideNT : NT) void lowfreq_kernel(
-    const CurveGeom* __restrict__ geom, const int32_t* __restrict__ list,
-    const CurveState* __restrict__ state, PointArrays pa, PlanParams pp, int kbegin,
-    void* __restrict__ out) {
-    constexpr int BT = WIDE ? kLowWideNT : NT;     // threads per block
-    __shared__ double red[BT / kWave][6];
-    constexpr int FPB = WIDE ? 1 : kLowPerBlock;   // frequencies per block
-    constexpr int LANES = WIDE ? BT : kWave;       // lanes per frequency
-    const int tid = threadIdx.x;
-    const int lane = tid % LANES;
-    const int c = list[blockIdx.x];
-    const CurveGeom& G = geom[c];
-    const CurveState& st = state[c];
-    int first = kbegin + (int)blockIdx.y * FPB;
-    do {
-        // frequency k is low if it and every frequency before it span fewer
-        // than kLowCycles cycles over the baseline (the leading run of the grid)
-        if (first >= G.nf) return;
-        if (fabs(G.f0 + (double)first * G.df) * st.tspan >= kLowCycles) return;
-        const int k = first + tid / LANES;
-        bool active = k < G.nf;
-        for (int q = first; q <= k && active; ++q)
-            active = fabs(G.f0 + (double)q * G.df) * st.tspan < kLowCycles;
-        // uniform per frequency: whole waves (or the block) exit; later groups
-        // of this block lie further along the grid, past the run as well
-        if (!active) return;
-        lowfreq_one<OUT, WIDE, BT, LANES>(G, st, pa, pp, k, tid, lane, G.n_obs, red, out);
-        first += (int)gridDim.y * FPB;
-    } while (LOOP);
-}
-
-// Wide curves with a WideAux record: grid (wide curve, frequency, part);
-// each of the kLowSplit workgroups of a low frequency sums one slice of the
-// points and stores its six FP64 sums in the record; the last to finish adds
-// the slices in order and forms the power.  Frequencies past the low run exit at once.
-template <int OUT>
-__global__ __launch_bounds__(kLowWideNT) void lowfreq_split_kernel(
-    const CurveGeom* __restrict__ geom, const int32_t* __restrict__ list,
-    const CurveState* __restrict__ state, PointArrays pa, PlanParams pp,
-    WideAux* __restrict__ aux, void* __restrict__ out) {
-    __shared__ double red[kLowWideNT / kWave][6];
-    const int tid = threadIdx.x;
-    const int k = blockIdx.y;
-    const int c = list[blockIdx.x];
-    const CurveGeom& G = geom[c];
-    const CurveState& st = state[c];
-    if (k >= min(G.nf, kLowMax)) return;
-    const double f = G.f0 + (double)k * G.df;
-    if (fabs(f) * st.tspan >= kLowCycles) return;   // the test of lowfreq_kernel<OUT, true>
-    const int N = G.n_obs;
-    const int per = (N + kLowSplit - 1) / kLowSplit;
-    const int j0 = (int)blockIdx.z * per;
-    const int j1 = min(N, j0 + per);
-    double acc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int j = j0 + tid; j < j1; j += kLowWideNT) {
-        const double x = f * pa.dt[G.pts + j];
-        double sn, cs;
-        sincospi(2.0 * (x - rint(x)), &sn, &cs);
-        const double w = pa.w[G.pts + j], yw = pa.yw[G.pts + j];
-        acc[0] += w * cs;
-        acc[1] += w * sn;
-        acc[2] += w * (cs * cs - sn * sn);
-        acc[3] += w * (2.0 * cs * sn);
-        acc[4] += yw * cs;
-        acc[5] += yw * sn;
-    }
+    };
+    if (N <= kLowShort) {
+        // few points: a wave takes four groups, 16 lanes over the points of
+        // each (a workgroup for each group spends its time on its barriers)
+        constexpr int kRun = 4 * kLowGroup;
+        double(*const rw)[kLowSums] = red[wv];
+        for (int t = first_task * WAVES + wv; t * kRun < kl; t += nblocks * WAVES) {
+            double acc[kLowSums];
 #pragma unroll
-    for (int q = 0; q < 6; ++q) acc[q] = wave_sum(acc[q]);
-    const int wv = tid / kWave;
-    if ((tid & (kWave - 1)) == 0)
-        for (int q = 0; q < 6; ++q) red[wv][q] = acc[q];
-    __syncthreads();
-    if (tid != 0) return;
-    for (int w = 1; w < kLowWideNT / kWave; ++w)
-        for (int q = 0; q < 6; ++q) acc[q] += red[w][q];
-    WideAux& X = aux[blockIdx.x];
-    for (int q = 0; q < 6; ++q) X.low[k][blockIdx.z][q] = acc[q];
-    __threadfence();
-    if (atomicAdd(&X.low_done[k], 1) != kLowSplit - 1) return;
-    __threadfence();
-    // the slices in order, so the sum does not depend on which finished first
-    double sm[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int z = 0; z < kLowSplit; ++z)
-        for (int q = 0; q < 6; ++q)
-            sm[q] += __hip_atomic_load(&X.low[k][z][q], __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-    const double P = gls_power(sm[0], sm[1], sm[2], sm[3], sm[4], sm[5], st.yy, st.ybar,
-                               pp.mode, pp.reg_c, pp.reg_s);
-    if (OUT == 0) ((float*)out)[G.out + k] = (float)P;
-    else ((double*)out)[G.out + k] = P;
+            for (int q = 0; q < kLowSums; ++q) acc[q] = 0.0;
+            const int g = lane >> 4;
+            low_points(G, pa, t * kRun + g * kLowGroup, lane & 15, N, 16, acc);
+            const int first = lane_sum_scatter<kLowSums, 8>(acc, lane);
+            if ((lane & 1) == 0) {
+#pragma unroll
+                for (int q = 0; q < kLowSums / 8; ++q) rw[g][first + q] = acc[q];
+            }
+            // (one wave: its LDS accesses are in order)
+            __builtin_amdgcn_wave_barrier();
+            const int k = t * kRun + lane;
+            if (lane < kRun && k < kl) store(k, &rw[lane / kLowGroup][6 * (lane % kLowGroup)]);
+            __builtin_amdgcn_wave_barrier();
+        }
+        return;
+    }
+    WideAux* const X = (wide && aux) ? aux + wi : nullptr;
+    // slices: of at least kLowSlice points, within the record's slots
+    int S = 1;
+    if (X)
+        while (2 * S * ngroups <= kLowSlots && 2 * S * kLowSlice <= N) S *= 2;
+    const int per = (N + S - 1) / S;
+    for (int task = first_task; task < ngroups * S; task += nblocks) {
+        const int g = task / S, z = task % S;
+        const int k0 = g * kLowGroup;
+        double acc[kLowSums];
+#pragma unroll
+        for (int q = 0; q < kLowSums; ++q) acc[q] = 0.0;
+        low_points(G, pa, k0, z * per + tid, min(N, (z + 1) * per), kLowNT, acc);
+        const int first = lane_sum_scatter<kLowSums, 32>(acc, lane);
+        if ((lane & 7) == 0) {
+#pragma unroll
+            for (int q = 0; q < kLowSums / 8; ++q) red[wv][0][first + q] = acc[q];
+        }
+        __syncthreads();
+        if (tid < kLowSums) {
+            double v = red[0][0][tid];
+#pragma unroll
+            for (int q = 1; q < WAVES; ++q) v += red[q][0][tid];
+            red[0][0][tid] = v;
+            if (S > 1) agent_publish(&X->low[task][tid], v);
+        }
+        __syncthreads();
+        bool done = true;
+        if (S > 1) {
+            if (tid == 0) last = atomicAdd(&X->low_done[g], 1) == S - 1;
+            __syncthreads();
+            done = last != 0;
+            if (done) {
+                // the slices in order, so the sum does not depend on which finished first
+                if (tid < kLowSums) {
+                    // (two slices or more: loads in flight four at a time)
+                    double v = 0.0;
+                    for (int q = 0; q < S; q += 4) {
+                        double u[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            u[i] = agent_load(&X->low[g * S + min(q + i, S - 1)][tid]);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            if (q + i < S) v += u[i];
+                    }
+                    red[0][0][tid] = v;
+                }
+                __syncthreads();
+            }
+        }
+        if (done && tid < kLowGroup && k0 + tid < kl) store(k0 + tid, &red[0][0][6 * tid]);
+        __syncthreads();   // red and last are reused by the next task
+    }
 }
 
 }  // namespace
 
-hipError_t launch_lowfreq(const CurveGeom* d_geom, const int32_t* small, int nsmall,
-                          const int32_t* wide, int nwide, const CurveState* state,
-                          PointArrays pa, const PlanParams& pp, void* power, int out_f64,
-                          WideAux* aux, hipStream_t s) {
-    // the first kLowMax frequencies: one group per block; any further ones
-    // (fine grids): a few looping blocks per curve, which exit at once when
-    // the low run ends before kLowMax
-    constexpr int kMoreGroups = 4;
-#define GLS_LOW(OUTV, W, L, GRID, NTH, LIST, KB)                                                \
-    hipLaunchKernelGGL((lowfreq_kernel<OUTV, W, L>), GRID, dim3(NTH), 0, s, d_geom, LIST, state, \
-                       pa, pp, KB, power)
-    if (nsmall > 0) {
-        if (out_f64) {
-            GLS_LOW(1, false, false, dim3(nsmall, kLowGroups), NT, small, 0);
-            GLS_LOW(1, false, true, dim3(nsmall, kMoreGroups), NT, small, kLowMax);
-        } else {
-            GLS_LOW(0, false, false, dim3(nsmall, kLowGroups), NT, small, 0);
-            GLS_LOW(0, false, true, dim3(nsmall, kMoreGroups), NT, small, kLowMax);
-        }
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-    }
-    if (nwide > 0 && aux != nullptr) {
-        // the first kLowMax frequencies split over kLowSplit workgroups each
-        // (one accumulator slot per frequency in the record)
-        const dim3 grid(nwide, kLowMax, kLowSplit);
+hipError_t launch_lowfreq(const CurveGeom* d_geom, const int32_t* list, int nsmall, int nwide,
+                          const CurveState* state, PointArrays pa, const PlanParams& pp,
+                          void* power, int out_f64, WideAux* aux, hipStream_t s) {
+    // a workgroup a curve in large batches, up to 16 (four are busy at the
+    // common 5 frequencies per 1/baseline) where the device would be idle; 512
+    // for a wide curve's slices.  Launches within kMaxLaunchItems
+    const int bs = std::max(1, std::min(16, 2048 / std::max(nsmall, 1)));
+    constexpr int bw = kLowSlots;
+    constexpr int64_t kBlocks = kMaxLaunchItems / kLowNT;
+    int s0 = 0, w0 = 0;
+    while (s0 < nsmall || w0 < nwide) {
+        const int ns = (int)std::min<int64_t>(nsmall - s0, kBlocks / bs);
+        // wide curves follow the small ones in the list
+        const int nw = s0 + ns < nsmall ? 0
+                       : (int)std::min<int64_t>(nwide - w0, (kBlocks - (int64_t)ns * bs) / bw);
+        const int32_t* l = list + (ns > 0 ? s0 : nsmall + w0);
+        WideAux* const x = aux ? aux + w0 : nullptr;
+        const dim3 grid((unsigned)((int64_t)ns * bs + (int64_t)nw * bw));
+        if (ns + nw == 0) return hipErrorInvalidValue;
         if (out_f64)
-            hipLaunchKernelGGL((lowfreq_split_kernel<1>), grid, dim3(kLowWideNT), 0, s, d_geom,
-                               wide, state, pa, pp, aux, power);
+            hipLaunchKernelGGL((lowfreq_kernel<1>), grid, dim3(kLowNT), 0, s, d_geom, l, ns, bs,
+                               bw, state, pa, pp, x, power);
         else
-            hipLaunchKernelGGL((lowfreq_split_kernel<0>), grid, dim3(kLowWideNT), 0, s, d_geom,
-                               wide, state, pa, pp, aux, power);
-        hipError_t e = hipGetLastError();
+            hipLaunchKernelGGL((lowfreq_kernel<0>), grid, dim3(kLowNT), 0, s, d_geom, l, ns, bs,
+                               bw, state, pa, pp, x, power);
+        const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
-    } else if (nwide > 0) {
-        if (out_f64) GLS_LOW(1, true, false, dim3(nwide, kLowMax), kLowWideNT, wide, 0);
-        else GLS_LOW(0, true, false, dim3(nwide, kLowMax), kLowWideNT, wide, 0);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
+        s0 += ns;
+        w0 += nw;
     }
-    if (nwide > 0) {
-        if (out_f64) GLS_LOW(1, true, true, dim3(nwide, kMoreGroups), kLowWideNT, wide, kLowMax);
-        else GLS_LOW(0, true, true, dim3(nwide, kMoreGroups), kLowWideNT, wide, kLowMax);
-    }
-#undef GLS_LOW
-    return hipGetLastError();
+    return hipSuccess;
 }
 
 // one launch per 2^31 work-items of tiles

@@ -161,11 +161,12 @@ constexpr int kWidePrep = 16384;
 constexpr int kWideChunk = 2048;
 constexpr int kMaxBuckets = 4096;   // n2 / c1 <= 2^12
 constexpr double kLowCycles = 3.0;
-constexpr int kLowMax = 256;
-constexpr int kLowSplit = 8;
-// (the record also holds, per low frequency, the six FP64 sums of each of the
-// kLowSplit workgroups of the low-frequency kernel, which the last of them adds
-// in slice order, and how many of them are done, cleared at every execute)
+constexpr int kLowGroup = 4;     // low frequencies summed together by a workgroup
+constexpr int kLowSlice = 4096;  // least points of a slice of a wide curve
+constexpr int kLowSlots = 512;   // (group, slice) pairs a wide curve may have
+// (the record also holds the FP64 sums of each (group, slice) pair of the
+// low-frequency kernel, which the last workgroup of a group adds in slice
+// order, and how many of a group's slices are done, cleared at every execute)
 struct WideAux {
     double ymean;
     double s0inv;
@@ -174,8 +175,8 @@ struct WideAux {
     int32_t yy_done;    // scatter blocks finished (variance partials)
     int32_t pad;
     int32_t hist[2][kMaxBuckets];
-    double low[kLowMax][kLowSplit][6];   // per low frequency and slice: the six sums
-    int32_t low_done[kLowMax];
+    double low[kLowSlots][6 * kLowGroup];
+    int32_t low_done[kLowSlots / 2];   // (two slices or more: at most half the slots)
 };
 // Per-chunk partial reductions of a wide curve, one slot per chunk of
 // kWideChunk points, combined in chunk order by the last block to finish (so
@@ -242,13 +243,12 @@ hipError_t launch_dirsum(const CurveGeom* d_geom, const CurveState* state,
                          const PlanParams& pp, void* power, int out_f64,
                          hipStream_t s);
 // direct FP64 sums for a curve's lowest frequencies, f_k (t_max - t_min) <
-// kLowCycles (all of them), overwriting the NFFT powers there; with aux (one
-// WideAux per wide curve) a wide curve's first kLowMax such frequencies are
-// each summed by kLowSplit workgroups, any further ones by one workgroup
-hipError_t launch_lowfreq(const CurveGeom* d_geom, const int32_t* small, int nsmall,
-                          const int32_t* wide, int nwide, const CurveState* state,
-                          PointArrays pa, const PlanParams& pp, void* power, int out_f64,
-                          WideAux* aux, hipStream_t s);
+// kLowCycles (all of them), overwriting the NFFT powers there; list: nsmall
+// curves, then nwide ones, which split their points over workgroups when they
+// have records (aux)
+hipError_t launch_lowfreq(const CurveGeom* d_geom, const int32_t* list, int nsmall, int nwide,
+                          const CurveState* state, PointArrays pa, const PlanParams& pp,
+                          void* power, int out_f64, WideAux* aux, hipStream_t s);
 hipError_t launch_dirsum_custom(const CurveGeom* d_geom, const CurveState* state,
                                 const int32_t* tile_curve, const int32_t* tile_first,
                                 int ntiles, int ws, PointArrays pa, const PlanParams& pp,

@@ -714,7 +714,7 @@ int run_plan(gls_plan* P, const double* t, const void* a, const void* b, void* o
             }
         }
         if (P->kind == 0 && !P->pp.fp32_coords) {
-            GLS_HIP_TRY(launch_lowfreq(d_geom, d_prep, P->nprep_small, d_prep + P->nprep_small,
+            GLS_HIP_TRY(launch_lowfreq(d_geom, d_prep, P->nprep_small,
                                        P->ncurves - P->nprep_small, state, pa, pp, out,
                                        out_f64, aux, s));
             GLS_HIP_TRY(mark());

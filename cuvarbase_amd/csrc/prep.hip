@@ -353,11 +353,7 @@ __global__ __launch_bounds__(NT) void wide_clear_kernel(const CurveGeom* __restr
         X.hist[0][i] = 0;
         X.hist[1][i] = 0;
     }
-    for (int i = tid; i < kLowMax; i += NT) X.low_done[i] = 0;
-}
-
-__device__ __forceinline__ double agent_load(const double* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int i = tid; i < kLowSlots / 2; i += NT) X.low_done[i] = 0;
 }
 
 // wide_reduce_kernel: the reductions of phase A per chunk (time range; for
