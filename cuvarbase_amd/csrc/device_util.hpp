@@ -27,23 +27,37 @@ __device__ __forceinline__ T wave_sum(T v) {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
     return v;
 }
-template <typename T>
-__device__ __forceinline__ T wave_min(T v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        T u = __shfl_xor(v, o, kWave);
-        v = u < v ? u : v;
-    }
-    return v;
+// FP64 exchange within a row of 16 lanes by data-parallel moves (CTRL: their
+// control code) and a lane's value for the whole wave: on the vector ALU, where
+// a shuffle takes two passes of the LDS that all waves of a CU share
+template <int CTRL>
+__device__ __forceinline__ double row_move(double v) {
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true));
 }
-template <typename T>
-__device__ __forceinline__ T wave_max(T v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        T u = __shfl_xor(v, o, kWave);
-        v = u > v ? u : v;
-    }
-    return v;
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+// op over the wave (the same in every lane): pairs, quads, eights and rows,
+// then the four rows
+template <class Op>
+__device__ __forceinline__ double wave_fold(double v, Op op) {
+    v = op(v, row_move<0xB1>(v));    // lanes i and i ^ 1
+    v = op(v, row_move<0x4E>(v));    // i ^ 2
+    v = op(v, row_move<0x141>(v));   // mirrored halves of a row
+    v = op(v, row_move<0x140>(v));   // mirrored rows
+    return op(op(lane_value(v, 0), lane_value(v, 16)), op(lane_value(v, 32), lane_value(v, 48)));
+}
+template <>
+__device__ __forceinline__ double wave_sum<double>(double v) {
+    return wave_fold(v, [](double x, double y) { return x + y; });
+}
+__device__ __forceinline__ double wave_min(double v) {
+    return wave_fold(v, [](double x, double y) { return fmin(x, y); });
+}
+__device__ __forceinline__ double wave_max(double v) {
+    return wave_fold(v, [](double x, double y) { return fmax(x, y); });
 }
 
 // Block-wide reductions for blockDim.x == NT (multiple of 64).  `scratch`
@@ -176,6 +190,19 @@ __device__ __forceinline__ double2 expi64_turn4(double y) {
 
 // exp(2 pi i r) for a phase r given in revolutions as FP64
 __device__ __forceinline__ float2 expi_rev(double r) { return expi_turn4(4.0 * r); }
+
+// number of leading low frequencies of a curve
+__device__ __forceinline__ int low_count(const CurveGeom& G, double tspan) {
+    auto low = [&](int k) { return fabs(G.f0 + (double)k * G.df) * tspan < kLowCycles; };
+    if (!low(0)) return 0;
+    if (!(tspan > 0.0)) return G.nf;
+    // the run ends near (kLowCycles / tspan - f0) / df, exactly where low() says
+    const double e = (kLowCycles / tspan - G.f0) / G.df;
+    int k = e < (double)G.nf ? max(1, (int)e) : G.nf;
+    while (k < G.nf && low(k)) ++k;
+    while (k > 1 && !low(k - 1)) --k;
+    return k;
+}
 
 // Buffer access to one curve's grid region (at most 3 grids of 2^24
 // complex64 cells, under 2^32 bytes): the base address and size live in a

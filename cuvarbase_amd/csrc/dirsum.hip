@@ -269,18 +269,6 @@ constexpr int kLowNT = 256;
 constexpr int kLowSums = 6 * kLowGroup;
 constexpr int kLowShort = 256;   // points up to which a wave sums alone
 
-// number of leading low frequencies of a curve
-__device__ __forceinline__ int low_count(const CurveGeom& G, double tspan) {
-    auto low = [&](int k) { return fabs(G.f0 + (double)k * G.df) * tspan < kLowCycles; };
-    if (!low(0)) return 0;
-    // the run ends near (kLowCycles / tspan - f0) / df, exactly where low() says
-    const double e = (kLowCycles / tspan - G.f0) / G.df;
-    int k = e < (double)G.nf ? max(1, (int)e) : G.nf;
-    while (k < G.nf && low(k)) ++k;
-    while (k > 1 && !low(k - 1)) --k;
-    return k;
-}
-
 // sums V values over lanes that differ in the bits HI, HI / 2 .. 1 of their
 // number: an exchange per value, but each step halves the values a lane holds
 // while their number is even.  Afterwards v[0 .. V/8) of a lane are the sums
@@ -349,12 +337,12 @@ __device__ __forceinline__ void low_points(const CurveGeom& G, const PointArrays
     }
 }
 
-// Workgroups: bs for each of the nsmall curves of the list, then bw for each of
-// the wide ones after them (those with a record in aux may split their points).
+// Workgroups: bs for each of the nsmall curves of the list (without a list, the
+// curves from first on), then bw for each of the wide ones after them (those with a record in aux may split their points).
 template <int OUT>
 __global__ __launch_bounds__(kLowNT) void lowfreq_kernel(
-    const CurveGeom* __restrict__ geom, const int32_t* __restrict__ list, int nsmall, int bs,
-    int bw, const CurveState* __restrict__ state, PointArrays pa, PlanParams pp,
+    const CurveGeom* __restrict__ geom, const int32_t* __restrict__ list, int first, int nsmall,
+    int bs, int bw, const CurveState* __restrict__ state, PointArrays pa, PlanParams pp,
     WideAux* __restrict__ aux, void* __restrict__ out) {
     constexpr int WAVES = kLowNT / kWave;
     __shared__ double red[WAVES][4][kLowSums];
@@ -365,12 +353,13 @@ __global__ __launch_bounds__(kLowNT) void lowfreq_kernel(
     const int bid = blockIdx.x;
     const bool wide = bid >= nsmall * bs;
     const int wi = wide ? (bid - nsmall * bs) / bw : 0;   // which of the wide curves
-    const int c = list[wide ? nsmall + wi : bid / bs];
+    const int ci = wide ? nsmall + wi : bid / bs;
+    const int c = list ? list[ci] : first + ci;
     const int first_task = wide ? (bid - nsmall * bs) % bw : bid % bs;
     const int nblocks = wide ? bw : bs;
     const CurveGeom& G = geom[c];
     const CurveState st = state[c];
-    const int kl = G.n_obs > 0 ? low_count(G, st.tspan) : 0;
+    const int kl = st.klow;
     const int ngroups = (kl + kLowGroup - 1) / kLowGroup;
     const int N = G.n_obs;
     auto store = [&](int k, const double* a) {
@@ -390,10 +379,10 @@ __global__ __launch_bounds__(kLowNT) void lowfreq_kernel(
             for (int q = 0; q < kLowSums; ++q) acc[q] = 0.0;
             const int g = lane >> 4;
             low_points(G, pa, t * kRun + g * kLowGroup, lane & 15, N, 16, acc);
-            const int first = lane_sum_scatter<kLowSums, 8>(acc, lane);
+            const int at = lane_sum_scatter<kLowSums, 8>(acc, lane);
             if ((lane & 1) == 0) {
 #pragma unroll
-                for (int q = 0; q < kLowSums / 8; ++q) rw[g][first + q] = acc[q];
+                for (int q = 0; q < kLowSums / 8; ++q) rw[g][at + q] = acc[q];
             }
             // (one wave: its LDS accesses are in order)
             __builtin_amdgcn_wave_barrier();
@@ -416,10 +405,10 @@ __global__ __launch_bounds__(kLowNT) void lowfreq_kernel(
 #pragma unroll
         for (int q = 0; q < kLowSums; ++q) acc[q] = 0.0;
         low_points(G, pa, k0, z * per + tid, min(N, (z + 1) * per), kLowNT, acc);
-        const int first = lane_sum_scatter<kLowSums, 32>(acc, lane);
+        const int at = lane_sum_scatter<kLowSums, 32>(acc, lane);
         if ((lane & 7) == 0) {
 #pragma unroll
-            for (int q = 0; q < kLowSums / 8; ++q) red[wv][0][first + q] = acc[q];
+            for (int q = 0; q < kLowSums / 8; ++q) red[wv][0][at + q] = acc[q];
         }
         __syncthreads();
         if (tid < kLowSums) {
@@ -476,16 +465,17 @@ hipError_t launch_lowfreq(const CurveGeom* d_geom, const int32_t* list, int nsma
         // wide curves follow the small ones in the list
         const int nw = s0 + ns < nsmall ? 0
                        : (int)std::min<int64_t>(nwide - w0, (kBlocks - (int64_t)ns * bs) / bw);
-        const int32_t* l = list + (ns > 0 ? s0 : nsmall + w0);
+        const int f = ns > 0 ? s0 : nsmall + w0;
+        const int32_t* l = list ? list + f : nullptr;
         WideAux* const x = aux ? aux + w0 : nullptr;
         const dim3 grid((unsigned)((int64_t)ns * bs + (int64_t)nw * bw));
         if (ns + nw == 0) return hipErrorInvalidValue;
         if (out_f64)
-            hipLaunchKernelGGL((lowfreq_kernel<1>), grid, dim3(kLowNT), 0, s, d_geom, l, ns, bs,
-                               bw, state, pa, pp, x, power);
+            hipLaunchKernelGGL((lowfreq_kernel<1>), grid, dim3(kLowNT), 0, s, d_geom, l, f, ns,
+                               bs, bw, state, pa, pp, x, power);
         else
-            hipLaunchKernelGGL((lowfreq_kernel<0>), grid, dim3(kLowNT), 0, s, d_geom, l, ns, bs,
-                               bw, state, pa, pp, x, power);
+            hipLaunchKernelGGL((lowfreq_kernel<0>), grid, dim3(kLowNT), 0, s, d_geom, l, f, ns,
+                               bs, bw, state, pa, pp, x, power);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         s0 += ns;

@@ -109,6 +109,8 @@ struct CurveState {
     double yy;
     double tspan;      // max t - min t
     double tmean;      // mean of the finite t (FP32-coordinate plans only)
+    int32_t klow;      // leading frequencies with |f| tspan < kLowCycles
+    int32_t pad;
 };
 
 // per-point workspace, indexed by CurveGeom::pts + j.  A node record holds a
@@ -151,13 +153,13 @@ bool pass1_tile_built(int n1, int c1);
 bool pass2_tile_built(int p2, int cr);
 
 // launchers (defined in the kernel translation units)
-// curves of more than kWidePrep points are prepared by 1024-thread blocks
-constexpr int kWidePrep = 16384;
-// For the NFFT method their point bucketing is spread over many blocks of
+// For the NFFT method the preparation of curves of more than kWidePrep points
+// (wide curves) is spread over many blocks of
 // kWideChunk points each (a counting pass and a scatter pass), with this
 // per-curve record in the workspace: the raw-input weight constants found by
 // the one-block reductions, the count of counting blocks done, and per node
 // set the bucket counts, turned into bucket cursors by the last counting block.
+constexpr int kWidePrep = 16384;
 constexpr int kWideChunk = 2048;
 constexpr int kMaxBuckets = 4096;   // n2 / c1 <= 2^12
 constexpr double kLowCycles = 3.0;
@@ -189,15 +191,18 @@ struct WidePart {
     double syy;          // sum of (y - ymean - ybar)^2/dy^2 (raw input, from the scatter)
     double pad;
 };
+// small: nsmall curves, followed in the same list by the nwide wide ones (wide);
 // aux: one WideAux per wide curve (NFFT method), or nullptr to prepare each
 // wide curve in one block; part: ceil(wide_max_obs / kWideChunk) WidePart
-// slots per wide curve; wide_max_obs: the largest n_obs in the wide list
+// slots per wide curve; wide_max_obs: the largest n_obs in the wide list;
+// max_buckets: the most buckets (n2 / c1) of a curve (NFFT method); in_order:
+// the list is 0, 1, 2 ..
 hipError_t launch_prep(const CurveGeom* d_geom, const int32_t* small, int nsmall,
                        const int32_t* wide, int nwide, CurveState* state,
                        const double* t, const void* a, const void* b,
                        PointArrays pa, int32_t* bkt, const PlanParams& pp,
                        int y_is_f32, WideAux* aux, WidePart* part, int wide_max_obs,
-                       hipStream_t s);
+                       int max_buckets, bool in_order, hipStream_t s);
 // work-items of one launch of the NFFT passes: the dispatch counts a grid's
 // work-items in 32 bits, so a size bucket with more goes out in several
 // launches over consecutive curves (max_launch_items(): this, or a smaller
@@ -243,8 +248,8 @@ hipError_t launch_dirsum(const CurveGeom* d_geom, const CurveState* state,
                          const PlanParams& pp, void* power, int out_f64,
                          hipStream_t s);
 // direct FP64 sums for a curve's lowest frequencies, f_k (t_max - t_min) <
-// kLowCycles (all of them), overwriting the NFFT powers there; list: nsmall
-// curves, then nwide ones, which split their points over workgroups when they
+// kLowCycles (all of them), overwriting the NFFT powers there; list (or
+// nullptr: 0, 1, 2 ..): nsmall curves, then nwide ones, which split their points over workgroups when they
 // have records (aux)
 hipError_t launch_lowfreq(const CurveGeom* d_geom, const int32_t* list, int nsmall, int nwide,
                           const CurveState* state, PointArrays pa, const PlanParams& pp,

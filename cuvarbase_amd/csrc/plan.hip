@@ -56,8 +56,9 @@ struct gls_plan {
     // host image of the descriptors uploaded into workspace[0 .. meta.size())
     std::vector<char> meta;
     size_t off_geom = 0, off_bgeom = 0, off_tiles = 0, off_prep = 0;
-    std::vector<int32_t> prep_list;   // curves prepared by 256-thread blocks, then wide ones
+    std::vector<int32_t> prep_list;   // curves prepared by one workgroup, then wide ones
     int nprep_small = 0;
+    bool prep_in_order = false;       // prep_list is 0, 1, 2 ..
     size_t off_state = 0, off_nd0 = 0, off_nd1 = 0, off_nd2 = 0,
            off_w = 0, off_yw = 0, off_dt = 0, off_bkt = 0,
            off_grid = 0;
@@ -66,6 +67,7 @@ struct gls_plan {
     size_t off_wide = 0, off_wpart = 0;
     int nwide_aux = 0;
     int wide_max_obs = 0;
+    int max_buckets = 0;   // most buckets of a curve's pass-1 column blocks
     size_t ws_bytes = 0;
     int64_t total_out = 0;
     // optional per-stage timing (events recorded between launches)
@@ -320,7 +322,9 @@ int plan_nfft_geometry(gls_plan* P, int ngrids, Layout& L, int64_t total_pts,
             // bucket offsets in entry order, 2 (nb + 1) per curve, so that
             // pass 1 finds a curve's from its place in the entry alone
             G.bkt = bkt_ints;
-            bkt_ints += 2 * ((1 << G.p2) / G.c1 + 1);
+            const int nb = (1 << G.p2) / G.c1;
+            bkt_ints += 2 * (nb + 1);
+            P->max_buckets = std::max(P->max_buckets, nb);
             G.grid = (chunk > 0) ? acc : grid_total;
             acc += cells;
             grid_total += cells;
@@ -584,6 +588,7 @@ void reserve_meta(gls_plan* P, Layout& L, size_t nbcurves, size_t ntiles_ints) {
     P->nprep_small = (int)P->prep_list.size();
     for (int i = 0; i < P->ncurves; ++i)
         if (P->geom[i].n_obs > kWidePrep) P->prep_list.push_back(i);
+    P->prep_in_order = std::is_sorted(P->prep_list.begin(), P->prep_list.end());
     P->off_geom = L.take(sizeof(CurveGeom) * P->geom.size());
     P->off_prep = L.take(sizeof(int32_t) * P->prep_list.size());
     P->off_bgeom = L.take(sizeof(CurveGeom) * nbcurves);
@@ -666,7 +671,7 @@ int run_plan(gls_plan* P, const double* t, const void* a, const void* b, void* o
     WidePart* wpart = P->nwide_aux > 0 ? (WidePart*)(base + P->off_wpart) : nullptr;
     GLS_HIP_TRY(launch_prep(d_geom, d_prep, P->nprep_small, d_prep + P->nprep_small,
                             P->ncurves - P->nprep_small, state, t, a, b, pa, bkt, pp, y_is_f32,
-                            aux, wpart, P->wide_max_obs, s));
+                            aux, wpart, P->wide_max_obs, P->max_buckets, P->prep_in_order, s));
     GLS_HIP_TRY(mark());
     if (P->pp.method == GLS_METHOD_NFFT) {
         // fork the buckets over the caller's and the auxiliary streams (not
@@ -714,7 +719,7 @@ int run_plan(gls_plan* P, const double* t, const void* a, const void* b, void* o
             }
         }
         if (P->kind == 0 && !P->pp.fp32_coords) {
-            GLS_HIP_TRY(launch_lowfreq(d_geom, d_prep, P->nprep_small,
+            GLS_HIP_TRY(launch_lowfreq(d_geom, P->prep_in_order ? nullptr : d_prep, P->nprep_small,
                                        P->ncurves - P->nprep_small, state, pa, pp, out,
                                        out_f64, aux, s));
             GLS_HIP_TRY(mark());
