@@ -188,8 +188,16 @@ __device__ __forceinline__ double2 expi64_turn4(double y) {
     return make_double2((q + 1u) & 2u ? -cs : cs, q & 2u ? -sn : sn);
 }
 
-// exp(2 pi i r) for a phase r given in revolutions as FP64
-__device__ __forceinline__ float2 expi_rev(double r) { return expi_turn4(4.0 * r); }
+// exp(2 pi i r) for a phase r given in revolutions as FP64: the integer part
+// is removed in FP64 (r - rint(r) in [-1/2, 1/2]) and only the reduced phase
+// is evaluated in FP32.  The plain transforms use it: multi-harmonic fits near
+// a singular normal matrix turn any other rounding into another power.
+__device__ __forceinline__ float2 expi_rev(double r) {
+    const float rr = (float)(r - rint(r));
+    float s, c;
+    sincospif(2.0f * rr, &s, &c);
+    return make_float2(c, s);
+}
 
 // number of leading low frequencies of a curve
 __device__ __forceinline__ int low_count(const CurveGeom& G, double tspan) {

@@ -29,11 +29,27 @@ int hip_fail(hipError_t e, const char* what);
 bool initialised();
 int require_init();
 
-// Asynchronous host-to-device copy of a plan's descriptors through the
-// library's page-locked staging ring (allocated by gls_init): the source is
-// copied into the ring on the host and the DMA reads the ring, so the call
-// never waits on the runtime's shared pageable staging buffer.  Falls back to
-// a plain hipMemcpyAsync for blocks larger than half the ring.
+// Descriptors as a launch argument (the first of its kernel), at most what the
+// runtime takes beside the other arguments; device code reads them where the
+// arguments lie, since indexing the parameter would copy it to scratch memory.
+constexpr int kMetaArgWords = 224;
+struct MetaArg {
+    int4 w[kMetaArgWords];
+};
+#if defined(__HIP_DEVICE_COMPILE__)
+__device__ inline const int4* meta_arg_words() {
+    return (const int4*)__builtin_amdgcn_kernarg_segment_ptr();
+}
+#else
+__device__ inline const int4* meta_arg_words() { return nullptr; }
+#endif
+
+// Asynchronous host-to-device copy of a plan's descriptors: as launch arguments
+// where they fit, else through the library's page-locked staging ring
+// (allocated by gls_init): the source is copied into the ring on the host and
+// a kernel reads the ring, so the call never waits on the runtime's shared
+// pageable staging buffer.  Falls back to a plain hipMemcpyAsync for blocks
+// larger than half the ring.
 hipError_t upload_async(void* dst, const void* src, size_t bytes, hipStream_t s);
 
 // Device address and size of the static scratch array of the current device
@@ -196,13 +212,16 @@ struct WidePart {
 // wide curve in one block; part: ceil(wide_max_obs / kWideChunk) WidePart
 // slots per wide curve; wide_max_obs: the largest n_obs in the wide list;
 // max_buckets: the most buckets (n2 / c1) of a curve (NFFT method); in_order:
-// the list is 0, 1, 2 ..
+// the list is 0, 1, 2 ..; meta (or nullptr): the descriptors, meta_words 16-byte
+// words that are not in the workspace ws yet: the first launch takes them as an
+// argument and stores them there
 hipError_t launch_prep(const CurveGeom* d_geom, const int32_t* small, int nsmall,
                        const int32_t* wide, int nwide, CurveState* state,
                        const double* t, const void* a, const void* b,
                        PointArrays pa, int32_t* bkt, const PlanParams& pp,
                        int y_is_f32, WideAux* aux, WidePart* part, int wide_max_obs,
-                       int max_buckets, bool in_order, hipStream_t s);
+                       int max_buckets, bool in_order, const MetaArg* meta, int meta_words,
+                       char* ws, hipStream_t s);
 // work-items of one launch of the NFFT passes: the dispatch counts a grid's
 // work-items in 32 bits, so a size bucket with more goes out in several
 // launches over consecutive curves (max_launch_items(): this, or a smaller

@@ -649,7 +649,13 @@ int run_plan(gls_plan* P, const double* t, const void* a, const void* b, void* o
              int out_f64, int y_is_f32, void* ws, hipStream_t s, const double* freqs = nullptr,
              bool upload_meta = true, bool allow_fork = true) {
     char* base = (char*)ws;
-    if (upload_meta && !P->meta.empty())
+    // descriptors of a few curves ride on the first launch, others go ahead
+    MetaArg meta;
+    const bool ride = upload_meta && !P->meta.empty() && P->meta.size() <= sizeof(meta) &&
+                      (uintptr_t)base % 16 == 0;
+    if (ride)
+        std::memcpy(&meta, P->meta.data(), P->meta.size());
+    else if (upload_meta && !P->meta.empty())
         GLS_HIP_TRY(upload_async(base, P->meta.data(), P->meta.size(), s));
     const CurveGeom* d_geom = (const CurveGeom*)(base + P->off_geom);
     const CurveGeom* d_bgeom = (const CurveGeom*)(base + P->off_bgeom);
@@ -671,7 +677,8 @@ int run_plan(gls_plan* P, const double* t, const void* a, const void* b, void* o
     WidePart* wpart = P->nwide_aux > 0 ? (WidePart*)(base + P->off_wpart) : nullptr;
     GLS_HIP_TRY(launch_prep(d_geom, d_prep, P->nprep_small, d_prep + P->nprep_small,
                             P->ncurves - P->nprep_small, state, t, a, b, pa, bkt, pp, y_is_f32,
-                            aux, wpart, P->wide_max_obs, P->max_buckets, P->prep_in_order, s));
+                            aux, wpart, P->wide_max_obs, P->max_buckets, P->prep_in_order,
+                            ride ? &meta : nullptr, (int)(P->meta.size() / 16), base, s));
     GLS_HIP_TRY(mark());
     if (P->pp.method == GLS_METHOD_NFFT) {
         // fork the buckets over the caller's and the auxiliary streams (not

@@ -78,7 +78,7 @@ __device__ __forceinline__ int prep_cell(double dt, int g, const CurveGeom& G, i
 
 // band-centring modulation exp(2 pi i g Fc dt): the phase reduced in FP64
 // before the FP32 sine and cosine, or with F32 formed and reduced in FP32
-template <bool F32>
+template <int KIND, bool F32>
 __device__ __forceinline__ float2 prep_phase(double dt, int g, double Fc) {
     if (F32) {
         float r = (float)g * ((float)Fc * (float)dt);
@@ -87,7 +87,8 @@ __device__ __forceinline__ float2 prep_phase(double dt, int g, double Fc) {
         sincospif(2.0f * r, &sn, &cs);
         return make_float2(cs, sn);
     }
-    return expi_rev((double)g * (Fc * dt));
+    if (KIND == 2) return expi_rev((double)g * (Fc * dt));
+    return expi_turn4(4.0 * ((double)g * (Fc * dt)));
 }
 
 // weights of a point as FP64: (w, yw) for lomb, (-, y) for nfft
@@ -129,7 +130,7 @@ __device__ __forceinline__ void prep_emit(const PointArrays& pa, const CurveGeom
         double yc;
         const int U = prep_cell<F32>(dt, g, G, m, yc);
         const float fr = (float)(yc - floor(yc));
-        const float2 e = prep_phase<F32>(dt, g, Fc);
+        const float2 e = prep_phase<KIND, F32>(dt, g, Fc);
         const int pos = cursor(g - 1, (U & (n2 - 1)) >> lc1);
         const int64_t o = G.pts + pos;
         auto rec = [&](double s) {
@@ -196,8 +197,26 @@ __device__ __forceinline__ void block_fold(const double* part, int lane, double 
     for (int q = 0; q < NQ; ++q) v[q] = lane_value(x, 8 * q);
 }
 
-// One workgroup per curve (list[blockIdx.x]; without a list, curve blockIdx.x,
-// whose geometry then loads at once).  A thread keeps kPrepPts points
+// The descriptors of a launch: already in the workspace, or (META) in its own
+// arguments, from where the first workgroup also stores them for the kernels
+// that follow (one launch less than an upload of its own).
+template <bool META>
+struct MetaIn {};
+template <>
+struct MetaIn<true> {
+    MetaArg arg;
+};
+template <bool META>
+__device__ __forceinline__ const char* meta_base(char* ws, int words, int nt) {
+    if (!META) return ws;
+    const int4* const w = meta_arg_words();
+    if (blockIdx.x == 0 && blockIdx.y == 0)
+        for (int i = threadIdx.x; i < words; i += nt) ((int4*)ws)[i] = w[i];
+    return (const char*)w;
+}
+
+// One workgroup per curve (number blockIdx.x of the list; in order, curve
+// blockIdx.x, whose geometry then loads at once).  A thread keeps kPrepPts points
 // in registers, so a curve of up to kPrepNT kPrepPts = 1,024 points is read
 // once; longer ones are read again, tile by tile, in each phase.  The sums of
 // phase A are folded together: one barrier for the time range and the weighted
@@ -211,9 +230,9 @@ __device__ __forceinline__ void block_fold(const double* part, int lane, double 
 // us.
 constexpr int kPrepNT = 512;
 constexpr int kPrepPts = 2;
-template <int KIND, bool F32>
-__global__ __launch_bounds__(kPrepNT, 6) void prep_kernel(const CurveGeom* __restrict__ geom,
-                                                       const int32_t* __restrict__ list,
+template <int KIND, bool F32, bool META>
+__global__ __launch_bounds__(kPrepNT, 6) void prep_kernel(MetaIn<META>, char* ws, int meta_words,
+                                                       int off_geom, int off_list, bool in_order,
                                                        CurveState* __restrict__ state,
                                                        const double* __restrict__ t,
                                                        const void* __restrict__ a,
@@ -228,8 +247,9 @@ __global__ __launch_bounds__(kPrepNT, 6) void prep_kernel(const CurveGeom* __res
     __shared__ double redyy[W];
     __shared__ int wsum[W];
     extern __shared__ int hist[];   // the buckets of both node sets
-    const int c = list ? list[blockIdx.x] : (int)blockIdx.x;
-    const CurveGeom G = geom[c];
+    const char* const desc = meta_base<META>(ws, meta_words, kPrepNT);
+    const int c = in_order ? (int)blockIdx.x : ((const int32_t*)(desc + off_list))[blockIdx.x];
+    const CurveGeom G = ((const CurveGeom*)(desc + off_geom))[c];
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1), wv = tid / kWave;
     const int N = G.n_obs;
@@ -388,10 +408,13 @@ __global__ __launch_bounds__(kPrepNT, 6) void prep_kernel(const CurveGeom* __res
 //
 // wide_clear_kernel (one block per wide curve) zeroes the record's counters
 // and accumulators at every execute.
-__global__ __launch_bounds__(NT) void wide_clear_kernel(const CurveGeom* __restrict__ geom,
-                                                        const int32_t* __restrict__ wide,
+template <bool META>
+__global__ __launch_bounds__(NT) void wide_clear_kernel(MetaIn<META>, char* ws, int meta_words,
+                                                        int off_geom, int off_wide,
                                                         WideAux* __restrict__ aux) {
-    const CurveGeom& G = geom[wide[blockIdx.x]];
+    const char* const desc = meta_base<META>(ws, meta_words, NT);
+    const int c = ((const int32_t*)(desc + off_wide))[blockIdx.x];
+    const CurveGeom& G = ((const CurveGeom*)(desc + off_geom))[c];
     WideAux& X = aux[blockIdx.x];
     const int tid = threadIdx.x;
     const int nb = (1 << G.p2) / G.c1;
@@ -659,17 +682,22 @@ hipError_t launch_prep_t(const CurveGeom* d_geom, const int32_t* small, int nsma
                          const int32_t* wide, int nwide, CurveState* state, const double* t,
                          const void* a, const void* b, PointArrays pa, int32_t* bkt,
                          const PlanParams& pp, int y_is_f32, WideAux* aux, WidePart* part,
-                         int wide_max_obs, int max_buckets, bool in_order, hipStream_t s) {
+                         int wide_max_obs, int max_buckets, bool in_order,
+                         const MetaArg* meta, int meta_words, char* ws, hipStream_t s) {
     const int kind = (pp.kind == 1) ? 2 : (pp.input_kind == GLS_INPUT_RAW ? 0 : 1);
     const int method = (pp.kind == 1) ? GLS_METHOD_NFFT : pp.method;
     const int yf = (pp.kind == 1) ? y_is_f32 : 0;
-#define GLS_PREP_LAUNCH(K, LIST, COUNT)                                                       \
-    hipLaunchKernelGGL((prep_kernel<K, F32>), dim3(COUNT), dim3(kPrepNT), lds, s, d_geom, LIST, \
-                       state, t, a, b, pa, bkt, pp.m, method, yf)
-#define GLS_PREP_KIND(LIST, COUNT)                   \
-    if (kind == 0) GLS_PREP_LAUNCH(0, LIST, COUNT);  \
-    else if (kind == 1) GLS_PREP_LAUNCH(1, LIST, COUNT); \
-    else GLS_PREP_LAUNCH(2, LIST, COUNT)
+    const int off_geom = (int)((const char*)d_geom - ws), off_list = (int)((const char*)small - ws);
+    MetaIn<true> in;
+    if (meta) in.arg = *meta;
+#define GLS_PREP_LAUNCH(K, M, IN)                                                             \
+    hipLaunchKernelGGL((prep_kernel<K, F32, M>), dim3(nblocks), dim3(kPrepNT), lds, s, IN, ws, \
+                       meta_words, off_geom, off_list, in_order, state, t, a, b, pa, bkt,    \
+                       pp.m, method, yf)
+#define GLS_PREP_KIND(M, IN)                   \
+    if (kind == 0) GLS_PREP_LAUNCH(0, M, IN);  \
+    else if (kind == 1) GLS_PREP_LAUNCH(1, M, IN); \
+    else GLS_PREP_LAUNCH(2, M, IN)
     // wide curves take the chunked kernels on the NFFT path, else the same one
     // workgroup as the others, which they follow in the list
     const bool split = aux != nullptr && part != nullptr && method == GLS_METHOD_NFFT &&
@@ -677,14 +705,24 @@ hipError_t launch_prep_t(const CurveGeom* d_geom, const int32_t* small, int nsma
     const int nblocks = nsmall + (split ? 0 : nwide);
     const size_t lds = sizeof(int) * (kind == 2 ? 1 : 2) * (size_t)max_buckets;
     if (nblocks > 0) {
-        GLS_PREP_KIND(in_order ? nullptr : small, nblocks);
+        if (meta) {
+            GLS_PREP_KIND(true, in);
+        } else {
+            GLS_PREP_KIND(false, MetaIn<false>{});
+        }
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
 #undef GLS_PREP_KIND
 #undef GLS_PREP_LAUNCH
     if (nwide <= 0 || !split) return hipSuccess;
-    hipLaunchKernelGGL(wide_clear_kernel, dim3(nwide), dim3(NT), 0, s, d_geom, wide, aux);
+    const int off_wide = (int)((const char*)wide - ws);
+    if (meta && nblocks == 0)
+        hipLaunchKernelGGL((wide_clear_kernel<true>), dim3(nwide), dim3(NT), 0, s, in, ws,
+                           meta_words, off_geom, off_wide, aux);
+    else
+        hipLaunchKernelGGL((wide_clear_kernel<false>), dim3(nwide), dim3(NT), 0, s,
+                           MetaIn<false>{}, ws, meta_words, off_geom, off_wide, aux);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const dim3 grid((unsigned)((wide_max_obs + kWideChunk - 1) / kWideChunk), (unsigned)nwide);
@@ -711,12 +749,15 @@ hipError_t launch_prep(const CurveGeom* d_geom, const int32_t* small, int nsmall
                        const int32_t* wide, int nwide, CurveState* state, const double* t,
                        const void* a, const void* b, PointArrays pa, int32_t* bkt,
                        const PlanParams& pp, int y_is_f32, WideAux* aux, WidePart* part,
-                       int wide_max_obs, int max_buckets, bool in_order, hipStream_t s) {
+                       int wide_max_obs, int max_buckets, bool in_order,
+                         const MetaArg* meta, int meta_words, char* ws, hipStream_t s) {
     if (pp.fp32_coords && pp.kind == 0)
         return launch_prep_t<true>(d_geom, small, nsmall, wide, nwide, state, t, a, b, pa, bkt,
-                                   pp, y_is_f32, aux, part, wide_max_obs, max_buckets, in_order, s);
+                                   pp, y_is_f32, aux, part, wide_max_obs, max_buckets, in_order, meta,
+                                   meta_words, ws, s);
     return launch_prep_t<false>(d_geom, small, nsmall, wide, nwide, state, t, a, b, pa, bkt, pp,
-                                y_is_f32, aux, part, wide_max_obs, max_buckets, in_order, s);
+                                y_is_f32, aux, part, wide_max_obs, max_buckets, in_order, meta,
+                                   meta_words, ws, s);
 }
 
 }  // namespace gls

@@ -1,9 +1,12 @@
 // Context, errors, streams, events and memory of libgls.so (C ABI).
+#include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <deque>
 #include <mutex>
+#include <thread>
 #include <vector>
 
 #include "gls_internal.hpp"
@@ -28,21 +31,27 @@ hipStream_t g_aux[kAuxStreams] = {};
 constexpr int kMaxDevices = 64;
 void* g_scratch[kMaxDevices] = {};   // device address of `scratch`, per device
 
-// Page-locked staging ring of the descriptor uploads: a byte ring with one
-// event per in-flight span; a span is reused only after its copy completed.
+// Page-locked staging ring of the descriptor uploads: a byte ring whose spans
+// are reused once their copy has read them.  The copy kernel itself reports
+// that, by storing the span's number in its slot of a page-locked flag array:
+// the caller's stream may be gone by the time the span is wanted again, and an
+// event recorded on a destroyed stream cannot be asked.
 constexpr size_t kStageBytes = size_t(16) << 20;
-constexpr int kStageEvents = 256;
+constexpr int kStageSlots = 256;
 struct StageSpan {
     size_t off, len;
-    int ev;
+    int slot;
+    uint32_t number;
 };
 struct StageRing {
     char* base = nullptr;
     char* dev = nullptr;   // the ring's device address
+    uint32_t* flags = nullptr;       // kStageSlots numbers of finished copies
+    uint32_t* flags_dev = nullptr;
     size_t head = 0;
+    uint32_t count = 0;    // spans handed out
     std::deque<StageSpan> inflight;
-    hipEvent_t ev[kStageEvents] = {};
-    std::vector<int> free_ev;
+    std::vector<int> free_slots;
 };
 std::mutex g_stage_mu;
 StageRing g_stage;
@@ -51,8 +60,9 @@ StageRing g_stage;
 int stage_setup() {
     if (g_stage.base) return GLS_OK;
     void* p = nullptr;
-    GLS_HIP_TRY(hipHostMalloc(&p, kStageBytes, hipHostMallocDefault));
-    std::memset(p, 0, kStageBytes);   // fault the pages in now, not inside a copy
+    GLS_HIP_TRY(hipHostMalloc(&p, kStageBytes + sizeof(uint32_t) * kStageSlots,
+                              hipHostMallocDefault));
+    std::memset(p, 0, kStageBytes + sizeof(uint32_t) * kStageSlots);   // fault the pages in now
     {
         void* d = nullptr;
         if (hipHostGetDevicePointer(&d, p, 0) != hipSuccess) {
@@ -61,29 +71,54 @@ int stage_setup() {
         }
         g_stage.dev = (char*)d;
     }
-    for (int i = 0; i < kStageEvents; ++i) {
-        hipError_t e = hipEventCreateWithFlags(&g_stage.ev[i], hipEventDisableTiming);
-        if (e != hipSuccess) {
-            for (int j = 0; j < i; ++j) (void)hipEventDestroy(g_stage.ev[j]);
-            (void)hipHostFree(p);
-            return hip_fail(e, "hipEventCreateWithFlags (staging ring)");
-        }
-    }
-    g_stage.free_ev.clear();
-    for (int i = kStageEvents - 1; i >= 0; --i) g_stage.free_ev.push_back(i);
+    g_stage.flags = (uint32_t*)((char*)p + kStageBytes);
+    g_stage.flags_dev = g_stage.dev ? (uint32_t*)(g_stage.dev + kStageBytes) : nullptr;
+    g_stage.free_slots.clear();
+    for (int i = kStageSlots - 1; i >= 0; --i) g_stage.free_slots.push_back(i);
     g_stage.inflight.clear();
     g_stage.head = 0;
     g_stage.base = (char*)p;
     return GLS_OK;
 }
 
+// after the device has been synchronised
 void stage_teardown() {
     std::lock_guard<std::mutex> lk(g_stage_mu);
     if (!g_stage.base) return;
-    for (auto& sp : g_stage.inflight) (void)hipEventSynchronize(g_stage.ev[sp.ev]);
-    for (auto& e : g_stage.ev) (void)hipEventDestroy(e);
     (void)hipHostFree(g_stage.base);
     g_stage = StageRing{};
+}
+
+// workgroups of a ring copy that are done, per slot (zero between copies)
+__device__ unsigned g_stage_done[kStageSlots];
+
+constexpr int kStageThreads = 256;
+__global__ __launch_bounds__(kStageThreads) void stage_copy_kernel(const uint4* __restrict__ src,
+                                                                   uint4* __restrict__ dst,
+                                                                   size_t n, int slot,
+                                                                   uint32_t number,
+                                                                   uint32_t* flag) {
+    for (size_t i = (size_t)blockIdx.x * kStageThreads + threadIdx.x; i < n;
+         i += (size_t)gridDim.x * kStageThreads)
+        dst[i] = src[i];
+    __syncthreads();   // every wave's words have been read
+    if (threadIdx.x != 0) return;
+    if (__hip_atomic_fetch_add(&g_stage_done[slot], 1u, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT) != gridDim.x - 1)
+        return;
+    // (the exchange's result is waited for before the flag is stored)
+    const unsigned was = __hip_atomic_exchange(&g_stage_done[slot], 0u, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("" ::"v"(was));
+    __hip_atomic_store(flag, number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// descriptors that fit into a launch's arguments need no staging: the kernel
+// stores its own argument
+__global__ __launch_bounds__(kMetaArgWords) void stage_arg_kernel(MetaArg meta, int words,
+                                                                  int4* __restrict__ dst) {
+    const int i = threadIdx.x;
+    if (i < words) dst[i] = meta_arg_words()[i];
 }
 // Copies by a kernel (loads and stores over the bus from the shader cores,
 // no DMA engine): the DMA path's hipMemcpyAsync has been measured holding the
@@ -148,47 +183,95 @@ void* device_address(const void* p) {
 
 }  // namespace
 
+namespace {
+
+bool is_capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
+bool stage_finished(const StageSpan& sp) {
+    return __atomic_load_n(&g_stage.flags[sp.slot], __ATOMIC_ACQUIRE) == sp.number;
+}
+
+// waits until a span's copy has read it: the device has a second to get there
+// by itself, then everything enqueued is waited for (which also reports a
+// device that is lost)
+hipError_t stage_wait(const StageSpan& sp) {
+    const auto t0 = std::chrono::steady_clock::now();
+    while (!stage_finished(sp)) {
+        if (std::chrono::steady_clock::now() - t0 > std::chrono::seconds(1))
+            return hipDeviceSynchronize();
+        std::this_thread::yield();
+    }
+    return hipSuccess;
+}
+
+}  // namespace
+
 hipError_t upload_async(void* dst, const void* src, size_t bytes, hipStream_t s) {
     if (bytes == 0) return hipSuccess;
+    if (bytes % 16 || (uintptr_t)dst % 16)
+        return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
+    // a few curves' descriptors go as launch arguments; while the stream is
+    // captured all do, in pieces (a graph replays its arguments, but the ring's
+    // bytes are reused)
+    if (bytes <= sizeof(MetaArg) || is_capturing(s)) {
+        for (size_t done = 0; done < bytes; done += sizeof(MetaArg)) {
+            const size_t len = std::min(sizeof(MetaArg), bytes - done);
+            MetaArg arg;
+            std::memcpy(&arg, (const char*)src + done, len);
+            hipLaunchKernelGGL(stage_arg_kernel, dim3(1), dim3(kMetaArgWords), 0, s, arg,
+                               (int)(len / 16), (int4*)((char*)dst + done));
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
     std::lock_guard<std::mutex> lk(g_stage_mu);
     StageRing& R = g_stage;
     const size_t need = (bytes + 255) / 256 * 256;
-    if (!R.base || need > kStageBytes / 2)
+    if (!R.base || !R.dev || need > kStageBytes / 2)
         return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
     auto release = [&](std::deque<StageSpan>::iterator it) {
-        R.free_ev.push_back(it->ev);
+        R.free_slots.push_back(it->slot);
         return R.inflight.erase(it);
     };
     // spans whose copies have finished, oldest first
-    while (!R.inflight.empty() && hipEventQuery(R.ev[R.inflight.front().ev]) == hipSuccess)
-        release(R.inflight.begin());
+    while (!R.inflight.empty() && stage_finished(R.inflight.front())) release(R.inflight.begin());
     const size_t off = (R.head + need <= kStageBytes) ? R.head : 0;
-    // wait for older copies still reading [off, off + need), and for a free event
+    // wait for older copies still reading [off, off + need), and for a free slot
     for (auto it = R.inflight.begin(); it != R.inflight.end();) {
         if (it->off < off + need && off < it->off + it->len) {
-            hipError_t e = hipEventSynchronize(R.ev[it->ev]);
+            const hipError_t e = stage_wait(*it);
             if (e != hipSuccess) return e;
             it = release(it);
         } else {
             ++it;
         }
     }
-    if (R.free_ev.empty()) {
-        hipError_t e = hipEventSynchronize(R.ev[R.inflight.front().ev]);
+    if (R.free_slots.empty()) {
+        const hipError_t e = stage_wait(R.inflight.front());
         if (e != hipSuccess) return e;
         release(R.inflight.begin());
     }
     std::memcpy(R.base + off, src, bytes);
-    // a kernel copy from the ring's mapped address (no DMA engine), or the
-    // DMA path when the ring has no device address
-    hipError_t e = R.dev ? kernel_copy(dst, R.dev + off, bytes, s)
-                         : hipMemcpyAsync(dst, R.base + off, bytes, hipMemcpyHostToDevice, s);
+    const int slot = R.free_slots.back();
+    const uint32_t number = ++R.count;
+    const size_t words = bytes / 16;
+    const unsigned blocks =
+        (unsigned)std::min<size_t>((words + kStageThreads - 1) / kStageThreads, 2048);
+    hipLaunchKernelGGL(stage_copy_kernel, dim3(blocks), dim3(kStageThreads), 0, s,
+                       (const uint4*)(R.dev + off), (uint4*)dst, words, slot, number,
+                       R.flags_dev + slot);
+    const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const int ev = R.free_ev.back();
-    e = hipEventRecord(R.ev[ev], s);
-    if (e != hipSuccess) return e;
-    R.free_ev.pop_back();
-    R.inflight.push_back({off, need, ev});
+    R.free_slots.pop_back();
+    R.inflight.push_back({off, need, slot, number});
     R.head = off + need;
     return hipSuccess;
 }

@@ -300,8 +300,8 @@ int gls_lomb_execute(gls_plan* plan, const double* t, const void* a,
  * event wait).  Nothing in the array needs clearing between calls: every
  * execute initialises what it reads.  Size buckets run in series on `stream`
  * (gls_plan_set_fork is ignored).  Calls no hipMalloc/hipFree; the
- * descriptors go up through the library's page-locked staging, allocated by
- * gls_init. */
+ * descriptors go up as launch arguments or through the library's page-locked
+ * staging, allocated by gls_init. */
 #define GLS_STATIC_SCRATCH_BYTES (128u << 20)
 int gls_lomb_execute_static(gls_plan* plan, const double* t, const void* a,
                             const void* b, float* power, void* stream);
