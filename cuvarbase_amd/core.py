@@ -9,7 +9,7 @@ one when the package is imported).
 """
 from __future__ import annotations
 
-from ._device import Stream, set_device, synchronize
+from ._device import BufferPool, Stream, set_device, synchronize
 
 # keyword arguments of every process and their defaults
 PROCESS_KEYWORDS = (("reader", None), ("nstreams", None), ("function_kwargs", None),
@@ -35,8 +35,14 @@ class GPUAsyncProcess(object):
         self.prepared_functions = {}
         self._keep_alive = []       # device objects used by enqueued work
         self._on_finish = []        # host steps that need the enqueued work done
+        self._pool = BufferPool()   # memory of the batches on stream 0, between runs
         if self.nstreams:
             self._create_streams(self.nstreams)
+
+    def __del__(self):
+        pool = getattr(self, "_pool", None)
+        if pool is not None:
+            pool.close()
 
     def _select_device(self):
         set_device(self.device)

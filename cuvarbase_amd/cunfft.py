@@ -329,9 +329,11 @@ class NFFTAsyncProcess(GPUAsyncProcess):
             df = 1.0 / (samples_per_peak * (np.max(t) - np.min(t)))
             items.append((t, y, minimum_frequency, df, int(nf)))
         m = max((self.get_m(it[4]) for it in items), default=self.m)
-        batch = NFFTBatch(items, sigma=self.sigma, m=m)
+        batch = NFFTBatch(items, sigma=self.sigma, m=m, pool=self._pool)
         flat, keep = batch.launch(self._stream(0))
-        self._keep_alive.append(keep)
+        # (the result too: its page-locked block must not return to the pool before
+        # finish, even if the caller drops it)
+        self._keep_alive.append((keep, flat))
         parts = batch.split(flat)
         if not self.use_double:
             return parts

@@ -62,6 +62,33 @@ def set_launch_items(items):
     _lib.call("gls_launch_items_set", C.c_int64(int(items)))
 
 
+# gls_curve as a NumPy record, for batches described as columns
+CURVE_DTYPE = np.dtype([("obs_offset", "i8"), ("n_obs", "i4"), ("nf", "i4"), ("f0", "f8"),
+                        ("df", "f8"), ("out_offset", "i8"), ("ybar", "f8"), ("yy", "f8")])
+# and gls_nfft_item (padded to whole 8 bytes)
+ITEM_DTYPE = np.dtype({"names": CURVE_DTYPE.names[:6],
+                       "formats": ["i8", "i4", "i4", "f8", "f8", "i8"],
+                       "offsets": [CURVE_DTYPE.fields[f][1] for f in CURVE_DTYPE.names[:6]],
+                       "itemsize": C.sizeof(_lib.gls_nfft_item)})
+assert CURVE_DTYPE.itemsize == C.sizeof(_lib.gls_curve)
+assert all(getattr(_lib.gls_nfft_item, f).offset == ITEM_DTYPE.fields[f][1]
+           for f in ITEM_DTYPE.names)
+
+
+def _records(items, struct, dtype):
+    """(ctypes array, count) of a list of structures or of an array of records."""
+    n = len(items)
+    if isinstance(items, np.ndarray):
+        buf = np.ascontiguousarray(items if n else np.zeros(1, dtype), dtype=dtype)
+        arr = (struct * max(n, 1)).from_address(buf.ctypes.data)
+        arr._gls_owner = buf
+        return arr, n
+    arr = (struct * max(n, 1))()
+    for i, c in enumerate(items):
+        arr[i] = c
+    return arr, n
+
+
 class Plan:
     """Owns a ``gls_plan`` handle."""
 
@@ -73,10 +100,7 @@ class Plan:
              grid_chunk_bytes=0, window=0, window_beta=0.0, point_capacity=0, precision=0,
              spread=0):
         _lib.init(0)
-        n = len(curves)
-        arr = (_lib.gls_curve * max(n, 1))()
-        for i, c in enumerate(curves):
-            arr[i] = c
+        arr, n = _records(curves, _lib.gls_curve, CURVE_DTYPE)
         prm = _lib.gls_params(sigma=float(sigma), m=int(m), mode=int(mode),
                               reg_c=float(reg_c), reg_s=float(reg_s),
                               input_kind=int(input_kind), method=int(method),
@@ -100,10 +124,7 @@ class Plan:
     @classmethod
     def nfft(cls, items, sigma, m):
         _lib.init(0)
-        n = len(items)
-        arr = (_lib.gls_nfft_item * max(n, 1))()
-        for i, c in enumerate(items):
-            arr[i] = c
+        arr, n = _records(items, _lib.gls_nfft_item, ITEM_DTYPE)
         h = C.c_void_p()
         _lib.call("gls_nfft_plan_create", C.byref(h), arr, C.c_int32(n), C.c_double(sigma),
                   C.c_int32(m))
@@ -245,45 +266,50 @@ class LombBatch:
         ``SPREAD_FIXED`` (integer fixed-point accumulation for every curve:
         bitwise reproducible results; slower than FP32 atomics on sparse
         curves, faster on dense ones)
+    pool : a BufferPool for the device and page-locked memory, if every copy
+        and execute of the batch runs on that pool's one stream
     """
 
     def __init__(self, data, freqs, sigma=2.0, m=8, mode=_lib.MODE_FLOATING_MEAN,
                  amplitude_prior=None, use_fft=True, use_double=False,
                  input_kind="raw", ybar=None, yy=None, custom_freqs=False,
                  grid_chunk_bytes=0, window=_lib.WINDOW_GAUSSIAN, window_beta=0.0,
-                 precision=_lib.PRECISION_FP64_COORDS, spread=_lib.SPREAD_AUTO):
+                 precision=_lib.PRECISION_FP64_COORDS, spread=_lib.SPREAD_AUTO, pool=None):
         if len(freqs) != len(data):
             raise ValueError("need one frequency grid per light curve")
         self.ncurves = len(data)
         self.use_double = bool(use_double)
         self.input_kind = _lib.INPUT_RAW if input_kind == "raw" else _lib.INPUT_WEIGHTED
         self.out_dtype = np.float64 if use_double else np.float32
+        self.pool = pool
         lam = 0.0 if amplitude_prior is None else float(amplitude_prior) ** -2
-        curves, obs, out = [], 0, 0
-        self.n_obs = np.empty(self.ncurves, dtype=np.int64)
-        self.nf = np.empty(self.ncurves, dtype=np.int64)
-        self.out_offsets = np.empty(self.ncurves, dtype=np.int64)
         self.custom = bool(custom_freqs)
-        for i, (d, fr) in enumerate(zip(data, freqs)):
-            if self.custom:
-                fr = np.asarray(fr, dtype=np.float64)
+        self.n_obs = np.fromiter((len(d[0]) for d in data), np.int64, self.ncurves)
+        curves = np.zeros(self.ncurves, dtype=CURVE_DTYPE)
+        if self.custom:
+            arrays = [np.asarray(fr, dtype=np.float64) for fr in freqs]
+            for fr in arrays:
                 if fr.ndim != 1 or len(fr) < 1 or not np.all(np.isfinite(fr)):
                     raise ValueError("custom frequencies must be a finite 1-D array")
-                f0, df, nf = 0.0, 1.0, len(fr)
-            else:
-                f0, df, nf = linear_grid(fr)
-            n = len(d[0])
-            c = _lib.gls_curve(obs_offset=obs, n_obs=n, nf=nf, f0=f0, df=df, out_offset=out,
-                               ybar=0.0 if ybar is None else float(ybar[i]),
-                               yy=1.0 if yy is None else float(yy[i]))
-            curves.append(c)
-            self.n_obs[i] = n
-            self.nf[i] = nf
-            self.out_offsets[i] = out
-            obs += n
-            out += nf
-        self.total_obs = obs
-        self.total_out = out
+            grids = [(0.0, 1.0, len(fr)) for fr in arrays]
+        else:
+            # (curves often share one grid)
+            grids, last, grid = [], None, None
+            for fr in freqs:
+                if fr is not last or grid is None:
+                    last, grid = fr, linear_grid(fr)
+                grids.append(grid)
+        for name, column in zip(("f0", "df", "nf"), zip(*grids)):
+            curves[name] = column
+        self.nf = curves["nf"].astype(np.int64)
+        self.out_offsets = np.cumsum(self.nf) - self.nf
+        curves["n_obs"] = self.n_obs
+        curves["obs_offset"] = np.cumsum(self.n_obs) - self.n_obs
+        curves["out_offset"] = self.out_offsets
+        curves["ybar"] = 0.0 if ybar is None else ybar
+        curves["yy"] = 1.0 if yy is None else yy
+        obs = self.total_obs = int(self.n_obs.sum())
+        self.total_out = int(self.nf.sum())
         if self.custom:
             method = _lib.METHOD_DIRECT_CUSTOM
             self._freqs = np.concatenate([np.asarray(f, dtype=np.float64) for f in freqs])
@@ -293,44 +319,41 @@ class LombBatch:
         self.plan = Plan.lomb(curves, sigma, m, mode, lam, lam, self.input_kind, method,
                               grid_chunk_bytes, window, window_beta, precision=precision,
                               spread=spread)
-        # host staging of the inputs
-        t = np.empty(obs, dtype=np.float64)
-        if self.input_kind == _lib.INPUT_RAW:
-            a = np.empty(obs, dtype=np.float64)
-            b = np.empty(obs, dtype=np.float64)
-        else:
-            a = np.empty(obs, dtype=np.float32)
-            b = np.empty(obs, dtype=np.float32)
-        o = 0
-        for d in data:
-            n = len(d[0])
-            t[o:o + n] = d[0]
-            a[o:o + n] = d[1]
-            b[o:o + n] = d[2]
-            o += n
-        self._host = (t, a, b)
+        # host staging of the inputs: t, a, b in one block, each at a multiple
+        # of 256 bytes, so that they go up in one copy
+        in_type = np.float64 if self.input_kind == _lib.INPUT_RAW else np.float32
+        row_t = -(-8 * obs // 256) * 256
+        row = -(-np.dtype(in_type).itemsize * obs // 256) * 256
+        self._rows = (0, row_t, row_t + row, row_t + 2 * row)
+        self._block = np.empty(max(self._rows[3], 1), dtype=np.uint8)
+        self._host = tuple(
+            self._block[o:o + np.dtype(dt).itemsize * obs].view(dt)
+            for o, dt in zip(self._rows, (np.float64, in_type, in_type)))
+        for j, dst in enumerate(self._host):
+            o = 0
+            for d, n in zip(data, self.n_obs.tolist()):
+                dst[o:o + n] = d[j]
+                o += n
         self.d_t = self.d_a = self.d_b = self.d_power = self.d_ws = self.d_freqs = None
 
     # ---- device side ---------------------------------------------------
     def allocate(self):
         t, a, b = self._host
-        self.d_t = DeviceArray(max(len(t), 1), np.float64)
-        self.d_a = DeviceArray(max(len(a), 1), a.dtype)
-        self.d_b = DeviceArray(max(len(b), 1), b.dtype)
-        self.d_power = DeviceArray(max(self.total_out, 1), self.out_dtype)
-        self.d_ws = DeviceArray(self.plan.workspace_bytes, np.uint8)
+        self.d_in = DeviceArray(len(self._block), np.uint8, pool=self.pool)
+        self.d_t, self.d_a, self.d_b = (
+            DeviceArray.part(self.d_in, o, len(x), x.dtype)
+            for o, x in zip(self._rows, (t, a, b)))
+        self.d_power = DeviceArray(max(self.total_out, 1), self.out_dtype, pool=self.pool)
+        self.d_ws = DeviceArray(self.plan.workspace_bytes, np.uint8, pool=self.pool)
         if self.custom:
-            self.d_freqs = DeviceArray(max(self.total_out, 1), np.float64)
+            self.d_freqs = DeviceArray(max(self.total_out, 1), np.float64, pool=self.pool)
         return self
 
     def upload(self, stream=None):
         if self.d_t is None:
             self.allocate()
-        t, a, b = self._host
-        if len(t):
-            self.d_t.set_async(t, stream=stream)
-            self.d_a.set_async(a, stream=stream)
-            self.d_b.set_async(b, stream=stream)
+        if self.total_obs:
+            self.d_in.set_async(self._block, stream=stream)
         if self.custom:
             self.d_freqs.set_async(self._freqs, stream=stream)
         return self
@@ -348,7 +371,7 @@ class LombBatch:
 
     def download_async(self, out=None, stream=None):
         if out is None:
-            out = pinned_empty(max(self.total_out, 1), self.out_dtype)
+            out = pinned_empty(max(self.total_out, 1), self.out_dtype, pool=self.pool)
         self.d_power.get_async(out, stream=stream, count=self.total_out)
         return out
 
@@ -380,35 +403,34 @@ class LombBatch:
 
     def topk(self, k, mask=None, stream=None):
         """Top-k (power, index) per curve from the device result."""
-        tp = DeviceArray(max(self.ncurves * k, 1), np.float32)
-        ti = DeviceArray(max(self.ncurves * k, 1), np.int32)
+        if self.use_double:
+            raise NotImplementedError("topk on f64 powers")
+        nk = self.ncurves * k
+        n = max(nk, 1)
+        top = DeviceArray(2 * n, np.float32, pool=self.pool)   # powers, then indices
         dmask = None
         if mask is not None:
             dmask = DeviceArray.to_device(np.ascontiguousarray(mask, dtype=np.uint8))
-        if self.use_double:
-            raise NotImplementedError("topk on f64 powers")
         _lib.call("gls_topk", self.plan.handle, self.d_ws.ptr, self.d_power.ptr,
-                  dmask.ptr if dmask is not None else None, C.c_int32(k), tp.ptr, ti.ptr,
-                  _handle(stream))
+                  dmask.ptr if dmask is not None else None, C.c_int32(k), top.ptr,
+                  top.ptr + 4 * n, _handle(stream))
         # read back on the stream of the top-k launch (the null stream does not
         # wait for a non-blocking stream)
-        n = max(self.ncurves * k, 1)
-        p = tp.get_async(pinned_empty(n, np.float32), stream=stream, count=n)
-        i = ti.get_async(pinned_empty(n, np.int32), stream=stream, count=n)
+        out = top.get_async(pinned_empty(2 * n, np.float32, pool=self.pool), stream=stream)
         if stream is None:
             _lib.call("gls_device_synchronize")
         else:
             _lib.call("gls_stream_synchronize", _handle(stream))
-        nk = self.ncurves * k
-        return (np.array(p[:nk]).reshape(self.ncurves, k),
-                np.array(i[:nk]).reshape(self.ncurves, k))
+        return (np.array(out[:nk]).reshape(self.ncurves, k),
+                np.array(out[n:n + nk].view(np.int32)).reshape(self.ncurves, k))
 
 
 class NFFTBatch:
     """Adjoint NFFTs sum_j y_j exp(2 pi i (f0 + k df) t_j), k < nf, of many items."""
 
-    def __init__(self, items, sigma=2.0, m=8):
-        # items: list of (t, y, f0, df, nf)
+    def __init__(self, items, sigma=2.0, m=8, pool=None):
+        # items: list of (t, y, f0, df, nf); pool: as LombBatch's
+        self.pool = pool
         descs, obs, out = [], 0, 0
         self.nf, self.out_offsets = [], []
         for (t, y, f0, df, nf) in items:
@@ -430,13 +452,16 @@ class NFFTBatch:
         """Enqueue upload, execute and download on ``stream``; returns the
         page-locked complex64 result (valid once the stream has completed) and
         the device buffers the enqueued work uses, to be kept alive until then."""
-        d_t = DeviceArray.to_device(self._t if len(self._t) else np.zeros(1), stream=stream)
-        d_y = DeviceArray.to_device(self._y if len(self._y) else np.zeros(1), stream=stream)
-        d_out = DeviceArray(max(2 * self.total_out, 1), np.float32)
-        d_ws = DeviceArray(self.plan.workspace_bytes, np.uint8)
+        pool = self.pool
+        d_t = DeviceArray.to_device(self._t if len(self._t) else np.zeros(1), stream=stream,
+                                    pool=pool)
+        d_y = DeviceArray.to_device(self._y if len(self._y) else np.zeros(1), stream=stream,
+                                    pool=pool)
+        d_out = DeviceArray(max(2 * self.total_out, 1), np.float32, pool=pool)
+        d_ws = DeviceArray(self.plan.workspace_bytes, np.uint8, pool=pool)
         _lib.call("gls_nfft_execute", self.plan.handle, d_t.ptr, d_y.ptr, C.c_int32(0),
                   d_out.ptr, d_ws.ptr, _handle(stream))
-        out = pinned_empty(max(2 * self.total_out, 1), np.float32)
+        out = pinned_empty(max(2 * self.total_out, 1), np.float32, pool=pool)
         d_out.get_async(out, stream=stream, count=2 * self.total_out)
         return out[: 2 * self.total_out].view(np.complex64), (d_t, d_y, d_out, d_ws, self.plan)
 
@@ -478,7 +503,8 @@ class MultiHarmonicBatch:
     (cuvarbase/lombscargle.py:235-293)."""
 
     def __init__(self, data, freqs, nharmonics=2, sigma=2.0, m=8, amplitude_prior=None,
-                 use_double=False):
+                 use_double=False, pool=None):
+        self.pool = pool   # as LombBatch's
         if not 1 <= int(nharmonics) <= 4:
             raise ValueError("nharmonics must be in [1, 4]")
         if len(freqs) != len(data):
@@ -489,11 +515,16 @@ class MultiHarmonicBatch:
         self.use_double = bool(use_double)
         self.out_dtype = np.float64 if use_double else np.float32
         lam = 0.0 if amplitude_prior is None else float(amplitude_prior) ** -2
-        items, curves, ts, ys = [], [], [], []
+        curves, ts, ys = [], [], []
+        harm = np.r_[1:H + 1, 1:2 * H + 1]
+        items = np.zeros(len(data) * 3 * H, dtype=ITEM_DTYPE)
         obs = out = pw = 0
         self.nf, self.out_offsets = [], []
-        for (t, y, dy), fr in zip(data, freqs):
-            f0, df, K = linear_grid(fr)
+        last, grid = None, None
+        for i, ((t, y, dy), fr) in enumerate(zip(data, freqs)):
+            if fr is not last or grid is None:   # (curves often share one grid)
+                last, grid = fr, linear_grid(fr)
+            f0, df, K = grid
             t = np.asarray(t, np.float64)
             y = np.asarray(y, np.float64)
             w = 1.0 / np.asarray(dy, np.float64) ** 2
@@ -504,15 +535,16 @@ class MultiHarmonicBatch:
             n = len(t)
             ts += [t, t]
             ys += [yw, w]
-            rows = [(obs, n) for _ in range(H)] + [(obs + n, n) for _ in range(2 * H)]
-            harm = list(range(1, H + 1)) + list(range(1, 2 * H + 1))
             curves.append(_lib.gls_mh_curve(sums_offset=out, out_offset=pw, nf=K, pad=0, yy=yy,
                                             ybar=float(np.sum(yw)), sum_w=float(np.sum(w)),
                                             lam=lam))
-            for (o, cnt), h in zip(rows, harm):
-                items.append(_lib.gls_nfft_item(obs_offset=o, n_obs=cnt, nf=K, f0=h * f0,
-                                                df=h * df, out_offset=out))
-                out += K
+            row = items[i * 3 * H:(i + 1) * 3 * H]
+            row["obs_offset"][:H] = obs
+            row["obs_offset"][H:] = obs + n
+            row["n_obs"], row["nf"] = n, K
+            row["f0"], row["df"] = harm * f0, harm * df
+            row["out_offset"] = out + K * np.arange(3 * H)
+            out += 3 * H * K
             self.nf.append(K)
             self.out_offsets.append(pw)
             obs += 2 * n
@@ -529,18 +561,19 @@ class MultiHarmonicBatch:
 
     def run(self, stream=None):
         s = stream or Stream()
-        d_t = DeviceArray.to_device(self._t, stream=s)
-        d_y = DeviceArray.to_device(self._y, stream=s)
-        d_c = DeviceArray.to_device(self._curves, stream=s)
-        d_sums = DeviceArray(max(2 * self.total_sums, 1), np.float32)
-        d_ws = DeviceArray(self.plan.workspace_bytes, np.uint8)
-        d_p = DeviceArray(max(self.total_out, 1), self.out_dtype)
+        pool = self.pool
+        d_t = DeviceArray.to_device(self._t, stream=s, pool=pool)
+        d_y = DeviceArray.to_device(self._y, stream=s, pool=pool)
+        d_c = DeviceArray.to_device(self._curves, stream=s, pool=pool)
+        d_sums = DeviceArray(max(2 * self.total_sums, 1), np.float32, pool=pool)
+        d_ws = DeviceArray(self.plan.workspace_bytes, np.uint8, pool=pool)
+        d_p = DeviceArray(max(self.total_out, 1), self.out_dtype, pool=pool)
         _lib.call("gls_nfft_execute", self.plan.handle, d_t.ptr, d_y.ptr, C.c_int32(0),
                   d_sums.ptr, d_ws.ptr, _handle(s))
         _lib.call("gls_mh_power", d_sums.ptr, d_c.ptr, C.c_int32(self.ncurves),
                   C.c_int32(self.nharmonics), C.c_int32(self.max_nf), d_p.ptr,
                   C.c_int32(1 if self.use_double else 0), _handle(s))
-        flat = pinned_empty(max(self.total_out, 1), self.out_dtype)
+        flat = pinned_empty(max(self.total_out, 1), self.out_dtype, pool=pool)
         d_p.get_async(flat, stream=s, count=self.total_out)
         s.synchronize()
         return [np.array(flat[o:o + n]) for o, n in zip(self.out_offsets, self.nf)]

@@ -40,7 +40,7 @@ from ._device import DeviceArray, pinned_zeros, _handle
 from .core import GPUAsyncProcess
 from .cunfft import NFFTAsyncProcess, NFFTMemory
 from .engine import LombBatch, Plan
-from .utils import weights, normalize_light_curves
+from .utils import weights, normalize_light_curves, centre_light_curves
 from .utils import autofrequency as utils_autofreq
 
 
@@ -546,7 +546,7 @@ class LombScargleAsyncProcess(GPUAsyncProcess):
         its Python layer never launches; the reference requires a linear grid
         (cuvarbase/lombscargle.py:939-940)."""
         self._ready(**kwargs)
-        data = normalize_light_curves(data)
+        data = centre_light_curves(data)
         if custom_freqs:
             if freqs is None:
                 raise ValueError("custom_freqs=True needs explicit frequencies")
@@ -585,6 +585,9 @@ class LombScargleAsyncProcess(GPUAsyncProcess):
         batch = self._launch_batch(data, grids, use_fft=use_fft, custom=custom, **kwargs)
         flat = batch.download_async(stream=self._stream(0)) if transfer_to_host else \
             pinned_zeros(max(batch.total_out, 1), batch.out_dtype)
+        # (its page-locked block must not return to the pool before finish, even if
+        # the caller drops it)
+        self._keep_alive.append(flat)
         return list(zip(grids, batch.split(flat)))
 
     def _run_multiharmonic(self, data, grids, use_fft=True, memory=None, **kwargs):
@@ -601,7 +604,7 @@ class LombScargleAsyncProcess(GPUAsyncProcess):
         batch = MultiHarmonicBatch(data, grids, nharmonics=self.nharmonics,
                                    sigma=self.nfft_proc.sigma, m=m,
                                    amplitude_prior=kwargs.get("amplitude_prior", None),
-                                   use_double=self.use_double)
+                                   use_double=self.use_double, pool=self._pool)
         return list(zip(grids, batch.run(stream=self._stream(0))))
 
     def _launch_batch(self, data, grids, use_fft=True, custom=False, **kwargs):
@@ -613,7 +616,7 @@ class LombScargleAsyncProcess(GPUAsyncProcess):
                                      kwargs.get("window", False)),
                           amplitude_prior=kwargs.get("amplitude_prior", None),
                           use_fft=use_fft, use_double=self.use_double, input_kind="raw",
-                          custom_freqs=custom, **self._window_config())
+                          custom_freqs=custom, pool=self._pool, **self._window_config())
         stream = self._stream(0)
         batch.upload(stream=stream)
         batch.execute(stream=stream)
@@ -639,7 +642,7 @@ class LombScargleAsyncProcess(GPUAsyncProcess):
         back) unless the run needs host powers (use_double, python_dir_sums,
         preallocated memory)."""
         self._ready(**kwargs)
-        data = normalize_light_curves(data)
+        data = centre_light_curves(data)
         grid = self._shared_grid(data, freqs, **kwargs)
         keep = np.ones(len(grid), dtype=bool) if ignore_freq_mask is None else \
             ~np.asarray(ignore_freq_mask, dtype=bool)
@@ -654,10 +657,9 @@ class LombScargleAsyncProcess(GPUAsyncProcess):
                 skip = None if ignore_freq_mask is None else \
                     np.tile(~keep, len(part)).astype(np.uint8)
                 top_p, top_i = batch.topk(1, mask=skip, stream=self._stream(0))
-                for curve, z, k in zip(part, top_p[:, 0], top_i[:, 0]):
-                    best.append(grid[k] if k >= 0 else np.nan)
-                    significance.append(self._significance(curve, float(z) if k >= 0 else np.nan,
-                                                           fmax))
+                k, z = top_i[:, 0], top_p[:, 0].astype(np.float64)
+                best.extend(np.where(k >= 0, grid[k], np.nan))
+                significance.extend(_significances(part, np.where(k >= 0, z, np.nan), fmax))
             else:
                 for curve, (_, p) in zip(part, self.run(part, freqs=grid, use_fft=use_fft,
                                                         **kwargs)):
@@ -679,24 +681,51 @@ def fap_baluev(t, dy, z, fmax, d_K=3, d_H=1, use_gamma=True):
     (cuvarbase/lombscargle.py:1115-1184), including the reference's form of
     the first exponent factor, (z/pi)^0.5 * (d-1) (:1177)."""
     t = np.asarray(t, dtype=np.float64)
-    N = len(t)
+    w = np.power(np.asarray(dy, dtype=np.float64), -2)
+    tbar = np.dot(w, t) / np.sum(w)
+    Dt = np.dot(w, np.power(t - tbar, 2)) / np.sum(w)
+    return _baluev(len(t), Dt, np.asarray(z, dtype=np.float64), fmax, d_K, d_H, use_gamma)
+
+
+def _baluev(N, Dt, z, fmax, d_K=3, d_H=1, use_gamma=True):
+    """fap_baluev of N points whose times have the weighted variance Dt (N, Dt
+    and z may be arrays)."""
     d = d_K - d_H
     N_K = N - d_K
     N_H = N - d_H
     g = (0.5 * N_H) ** (0.5 * (d - 1))
     if use_gamma:
         g = np.exp(gammaln(0.5 * N_H) - gammaln(0.5 * (N_K + 1)))
-    w = np.power(np.asarray(dy, dtype=np.float64), -2)
-    tbar = np.dot(w, t) / np.sum(w)
-    Dt = np.dot(w, np.power(t - tbar, 2)) / np.sum(w)
     Teff = np.sqrt(4 * np.pi * Dt)
     A = (2 * np.pi ** 1.5) * fmax * Teff
-    z = np.asarray(z, dtype=np.float64)
     eZ1 = (z / np.pi) ** 0.5 * (d - 1)
     eZ2 = (1 - z) ** (0.5 * (N_K - 1))
     tau = (g * A / (2 * np.pi)) * eZ1 * eZ2
     Psing = 1 - (1 - z) ** (0.5 * N_K)
     return 1 - Psing * np.exp(-tau)
+
+
+def _significances(data, z, fmax):
+    """1 - Baluev FAP of each curve's peak power z (NaN where z is not finite),
+    all curves at a time."""
+    n = np.array([len(c[0]) for c in data])
+    out = np.full(len(data), np.nan)
+    ok = np.isfinite(z)
+    if not ok.any() or not n.all():
+        ok &= n > 0
+        data = [c for c, use in zip(data, ok) if use]
+        z, n = z[ok], n[ok]
+        if len(data):
+            out[ok] = _significances(data, z, fmax)
+        return out
+    starts = np.cumsum(n) - n
+    t = np.concatenate([np.asarray(c[0], np.float64) for c in data])
+    w = np.concatenate([np.asarray(c[2], np.float64) for c in data]) ** -2.0
+    sw = np.add.reduceat(w, starts)
+    t = t - np.repeat(np.add.reduceat(w * t, starts) / sw, n)
+    Dt = np.add.reduceat(w * t * t, starts) / sw
+    out[ok] = 1. - _baluev(n[ok], Dt[ok], z[ok], fmax)
+    return out
 
 
 def lomb_scargle_simple(t, y, dy, **kwargs):

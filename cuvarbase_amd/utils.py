@@ -55,3 +55,30 @@ def normalize_light_curves(data):
             cols[j] = cols[j] - np.nanmean(cols[j])
         centred.append(tuple(cols))
     return centred
+
+
+def _columns_alike(col, lengths):
+    return all(type(c) is np.ndarray and c.ndim == 1 and c.dtype == np.float64 and len(c) == n
+               for c, n in zip(col, lengths))
+
+
+def centre_light_curves(data):
+    """``normalize_light_curves`` for many curves at a time: where every column
+    of every curve is a 1-D float64 array (and none is empty), the columns are
+    concatenated, centred together and handed out as views."""
+    data = list(data)
+    width = len(data[0]) if data else 0
+    lengths = [len(d[0]) for d in data] if width else []
+    if width < 2 or not all(lengths) or any(len(d) != width for d in data) or \
+            not all(_columns_alike(col, lengths) for col in zip(*data)):
+        return normalize_light_curves(data)
+    n = np.array(lengths)
+    ends = np.cumsum(n)
+    columns = [np.concatenate(col) for col in zip(*data)]
+    for j in (0, 1):
+        mean = np.add.reduceat(columns[j], ends - n) / n
+        for i in np.flatnonzero(np.isnan(mean)):
+            mean[i] = np.nanmean(data[i][j])
+        columns[j] -= np.repeat(mean, n)
+    bounds = list(zip((ends - n).tolist(), ends.tolist()))
+    return [tuple(c[a:b] for c in columns) for a, b in bounds]
