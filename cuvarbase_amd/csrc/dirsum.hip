@@ -263,8 +263,8 @@ __global__ __launch_bounds__(kDirNT) void dirsum_custom_kernel(
 // the power.  Measured, against a sine and cosine per point and frequency, one
 // wave per frequency (1,024 lanes x 8 workgroups for wide curves) and two
 // launches: 2,000 curves of 20-300 points 64 -> 31 us, one of 1,000 points 15
-// -> 6 us, 37 of 400-3,000 points 28 -> 12 us, 32 of 100-50,000 points 89 -> 28
-// us, one of 200,000 points 32 -> 17 us.
+// -> 6 us, 37 of 400-3,000 points 28 -> 12 us, 32 of 100-50,000 points 89 -> 23
+// us, one of 200,000 points 32 -> 13 us.
 constexpr int kLowNT = 256;
 constexpr int kLowSums = 6 * kLowGroup;
 constexpr int kLowShort = 256;   // points up to which a wave sums alone
@@ -346,6 +346,7 @@ __global__ __launch_bounds__(kLowNT) void lowfreq_kernel(
     WideAux* __restrict__ aux, void* __restrict__ out) {
     constexpr int WAVES = kLowNT / kWave;
     __shared__ double red[WAVES][4][kLowSums];
+    __shared__ double slices[8][kLowSums];
     __shared__ int last;
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
@@ -425,19 +426,23 @@ __global__ __launch_bounds__(kLowNT) void lowfreq_kernel(
             __syncthreads();
             done = last != 0;
             if (done) {
-                // the slices in order, so the sum does not depend on which finished first
+                // the slices in order, so the sum does not depend on which finished
+                // first: kLowParts threads a sum, then those
+                constexpr int kLowParts = 8;
+                static_assert(kLowParts * kLowSums <= kLowNT, "one slice and sum per thread");
+                const int part = tid / kLowSums, q = tid % kLowSums;
+                double v = 0.0;
+                if (part < kLowParts) {
+#pragma unroll 4
+                    for (int i = part; i < S; i += kLowParts)
+                        v += agent_load(&X->low[g * S + i][q]);
+                    slices[part][q] = v;
+                }
+                __syncthreads();
                 if (tid < kLowSums) {
-                    // (two slices or more: loads in flight four at a time)
-                    double v = 0.0;
-                    for (int q = 0; q < S; q += 4) {
-                        double u[4];
+                    v = 0.0;
 #pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            u[i] = agent_load(&X->low[g * S + min(q + i, S - 1)][tid]);
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            if (q + i < S) v += u[i];
-                    }
+                    for (int i = 0; i < kLowParts; ++i) v += slices[i][tid];
                     red[0][0][tid] = v;
                 }
                 __syncthreads();

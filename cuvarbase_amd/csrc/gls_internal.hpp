@@ -170,17 +170,17 @@ bool pass2_tile_built(int p2, int cr);
 
 // launchers (defined in the kernel translation units)
 // For the NFFT method the preparation of curves of more than kWidePrep points
-// (wide curves) is spread over many blocks of
-// kWideChunk points each (a counting pass and a scatter pass), with this
-// per-curve record in the workspace: the raw-input weight constants found by
-// the one-block reductions, the count of counting blocks done, and per node
-// set the bucket counts, turned into bucket cursors by the last counting block.
+// (wide curves) is spread over at most kWideBlocks blocks of kWideChunk points or
+// a multiple of it each (a reduction, a counting and a scatter pass), with this
+// per-curve record in the workspace: the raw-input weight constants and the bucket
+// counts of both node sets, one after the other.
 constexpr int kWidePrep = 16384;
-constexpr int kWideChunk = 2048;
+constexpr int kWideChunk = 1024;
+constexpr int kWideBlocks = 1024;
 constexpr int kMaxBuckets = 4096;   // n2 / c1 <= 2^12
 constexpr double kLowCycles = 3.0;
 constexpr int kLowGroup = 4;     // low frequencies summed together by a workgroup
-constexpr int kLowSlice = 4096;  // least points of a slice of a wide curve
+constexpr int kLowSlice = 2048;  // least points of a slice of a wide curve
 constexpr int kLowSlots = 512;   // (group, slice) pairs a wide curve may have
 // (the record also holds the FP64 sums of each (group, slice) pair of the
 // low-frequency kernel, which the last workgroup of a group adds in slice
@@ -188,29 +188,25 @@ constexpr int kLowSlots = 512;   // (group, slice) pairs a wide curve may have
 struct WideAux {
     double ymean;
     double s0inv;
-    int32_t done;       // counting blocks finished
-    int32_t red_done;   // reduction blocks finished
-    int32_t yy_done;    // scatter blocks finished (variance partials)
-    int32_t pad;
-    int32_t hist[2][kMaxBuckets];
+    int32_t hist[2 * kMaxBuckets];    // points per bucket, both node sets
+    int32_t taken[2 * kMaxBuckets];   // of those, slots that chunks have reserved
     double low[kLowSlots][6 * kLowGroup];
     int32_t low_done[kLowSlots / 2];   // (two slices or more: at most half the slots)
 };
-// Per-chunk partial reductions of a wide curve, one slot per chunk of
-// kWideChunk points, combined in chunk order by the last block to finish (so
-// the result does not depend on block timing).
+// Per-chunk partial reductions of a wide curve, one slot per chunk, combined in
+// chunk order (so the result does not depend on block timing): least t and -t;
+// raw input: sum and count of the finite y, sums of 1/dy^2 and of y/dy^2; last
+// two, FP32 coordinates only: sum and count of the finite t.  syy: sum of (y -
+// ymean - ybar)^2/dy^2 (raw input, from the counting pass).
 struct WidePart {
-    double tmin, tmax;   // time range
-    double st, ct;       // sum and count of the finite t (FP32 coordinates only)
-    double sy, cy;       // sum and count of the finite y (raw input)
-    double sw, swy;      // sum of 1/dy^2 and of y/dy^2 (raw input)
-    double syy;          // sum of (y - ymean - ybar)^2/dy^2 (raw input, from the scatter)
+    double v[8];
+    double syy;
     double pad;
 };
 // small: nsmall curves, followed in the same list by the nwide wide ones (wide);
 // aux: one WideAux per wide curve (NFFT method), or nullptr to prepare each
-// wide curve in one block; part: ceil(wide_max_obs / kWideChunk) WidePart
-// slots per wide curve; wide_max_obs: the largest n_obs in the wide list;
+// wide curve in one block; part: min(kWideBlocks,
+// ceil(wide_max_obs / kWideChunk)) WidePart slots per wide curve; wide_max_obs: the largest n_obs in the wide list;
 // max_buckets: the most buckets (n2 / c1) of a curve (NFFT method); in_order:
 // the list is 0, 1, 2 ..; meta (or nullptr): the descriptors, meta_words 16-byte
 // words that are not in the workspace ws yet: the first launch takes them as an

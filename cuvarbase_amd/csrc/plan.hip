@@ -375,7 +375,7 @@ int plan_nfft_geometry(gls_plan* P, int ngrids, Layout& L, int64_t total_pts,
         }
     if (P->nwide_aux > 0) {
         P->off_wide = L.take(sizeof(WideAux) * (size_t)P->nwide_aux);
-        const size_t nchunks = ((size_t)P->wide_max_obs + kWideChunk - 1) / kWideChunk;
+        const int nchunks = std::min(kWideBlocks, (P->wide_max_obs + kWideChunk - 1) / kWideChunk);
         P->off_wpart = L.take(sizeof(WidePart) * nchunks * (size_t)P->nwide_aux);
     }
     P->off_grid = L.take(sizeof(float2) * grid_elems);

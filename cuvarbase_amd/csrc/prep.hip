@@ -11,21 +11,21 @@
 //            of every point, in FP64 before the cast to FP32, then a counting
 //            sort of the points by pass-1 column block (so every pass-1 tile
 //            reads only the points that touch it); for curves of more than
-//            16,384 points this phase runs as a counting kernel and a scatter
-//            kernel over chunks of 2,048 points (LDS counts per chunk, one
-//            global atomic per bucket and chunk);
+//            16,384 points both phases run over chunks of 1,024 points, as a
+//            reduction, a counting and a scatter kernel (LDS counts per chunk,
+//            one global atomic per bucket and chunk);
 //            (direct method) the FP32 weights and FP64 time offsets.
 // With FP32 coordinates (GLS_PRECISION_FP32, for comparison with the
 // reference's arithmetic) t is rounded to FP32 after centring on its mean and
 // the time offset, cell coordinate and modulation phase of every point are
 // FP32 operations; everything else is unchanged.
+#include <algorithm>
+
 #include "device_util.hpp"
 
 namespace gls {
 
 namespace {
-
-constexpr int NT = 256;
 
 struct PrepVals {
     double t;
@@ -246,7 +246,7 @@ __global__ __launch_bounds__(kPrepNT, 6) void prep_kernel(MetaIn<META>, char* ws
     __shared__ double red[NQ * W];
     __shared__ double redyy[W];
     __shared__ int wsum[W];
-    extern __shared__ int hist[];   // the buckets of both node sets
+    extern __shared__ __align__(16) int hist[];   // the buckets of both node sets
     const char* const desc = meta_base<META>(ws, meta_words, kPrepNT);
     const int c = in_order ? (int)blockIdx.x : ((const int32_t*)(desc + off_list))[blockIdx.x];
     const CurveGeom G = ((const CurveGeom*)(desc + off_geom))[c];
@@ -399,279 +399,322 @@ __global__ __launch_bounds__(kPrepNT, 6) void prep_kernel(MetaIn<META>, char* ws
     }, true);
 }
 
-// Wide curves (more than kWidePrep points, NFFT method) are prepared by
-// kernels over chunks of kWideChunk points: blockIdx.y picks the curve
-// (wide[blockIdx.y], record aux[blockIdx.y], chunk partials
-// part[blockIdx.y * gridDim.x ..]), blockIdx.x its chunk.  The grid has the
-// same chunk count for every wide curve (that of the longest); chunks past a
-// curve's end are empty.
-//
-// wide_clear_kernel (one block per wide curve) zeroes the record's counters
-// and accumulators at every execute.
-template <bool META>
-__global__ __launch_bounds__(NT) void wide_clear_kernel(MetaIn<META>, char* ws, int meta_words,
-                                                        int off_geom, int off_wide,
-                                                        WideAux* __restrict__ aux) {
-    const char* const desc = meta_base<META>(ws, meta_words, NT);
-    const int c = ((const int32_t*)(desc + off_wide))[blockIdx.x];
-    const CurveGeom& G = ((const CurveGeom*)(desc + off_geom))[c];
-    WideAux& X = aux[blockIdx.x];
-    const int tid = threadIdx.x;
-    const int nb = (1 << G.p2) / G.c1;
-    if (tid == 0) {
-        X.done = 0;
-        X.red_done = 0;
-        X.yy_done = 0;
+// Wide curves (more than kWidePrep points, NFFT method) are prepared by three
+// kernels over chunks of their points: blockIdx.y picks the curve (number
+// blockIdx.y of the wide ones, record aux[blockIdx.y], chunk partials part[
+// blockIdx.y gridDim.x ..]), blockIdx.x its chunk.  A chunk is kWideChunk
+// points, or as many times that as leave at most kWideBlocks chunks (the chunks
+// of a curve depend on its own points alone, so its results are the same in any
+// batch).  The grid has as many chunks as the longest curve may need; those
+// past a curve's end do nothing.  A thread holds kWidePts points of a chunk of
+// kWideChunk in registers.  Nothing waits for a last block: what a chunk leaves is
+// folded by every block of the next kernel.  Bound by latency (a chain of loads,
+// folds and atomics, all chunks at a time) and the scatter by its 16-byte
+// records.  Measured (200,000 points), against chunks of 2,048, last blocks
+// behind fences and a clearing launch: reduction 23 -> 5 us, counting 17 -> 12,
+// scatter 34 -> 19.
+constexpr int kWideNT = 512;
+constexpr int kWidePts = kWideChunk / kWideNT;
+static_assert(kWidePts * kWideNT == kWideChunk, "whole points per thread");
+
+struct WideSpan {
+    int j0, j1;    // this block's points
+    int chunks;    // chunks of the curve
+    __device__ __forceinline__ explicit WideSpan(int N) {
+        constexpr int kAll = kWideChunk * kWideBlocks;
+        const int64_t len = (int64_t)kWideChunk * (((int64_t)N + kAll - 1) / kAll);
+        chunks = (int)((N + len - 1) / len);
+        j0 = (int)min((int64_t)N, blockIdx.x * len);
+        j1 = (int)min((int64_t)N, j0 + len);
     }
-    for (int i = tid; i < nb; i += NT) {
-        X.hist[0][i] = 0;
-        X.hist[1][i] = 0;
+    // f(j, u) for this thread's points, u their places in kWidePts registers; load
+    // fills the registers of a round (a span of one round is loaded once)
+    template <class L, class F>
+    __device__ __forceinline__ void each(L&& load, F&& f, bool loaded) const {
+        for (int base = j0; base < j1; base += kWideChunk) {
+            if (!(loaded && j1 - j0 <= kWideChunk)) load(base);
+#pragma unroll
+            for (int u = 0; u < kWidePts; ++u) {
+                const int j = base + u * kWideNT + (int)threadIdx.x;
+                if (j < j1) f(j, u);
+            }
+        }
     }
-    for (int i = tid; i < kLowSlots / 2; i += NT) X.low_done[i] = 0;
-}
+};
 
 // wide_reduce_kernel: the reductions of phase A per chunk (time range; for
 // raw input the sums of the finite y, of 1/dy^2 and y/dy^2; with FP32
 // coordinates the sum of the finite t), each chunk's partials into its slot;
-// the last block to finish combines the slots in chunk order and writes the
-// curve's state (tref, span, ybar; yy follows from the scatter) and the
-// weight constants of the record.
-template <int KIND, bool F32>
-__global__ __launch_bounds__(NT) void wide_reduce_kernel(const CurveGeom* __restrict__ geom,
-                                                         const int32_t* __restrict__ wide,
-                                                         CurveState* __restrict__ state,
-                                                         const double* __restrict__ t,
-                                                         const void* __restrict__ a,
-                                                         const void* __restrict__ b,
-                                                         WideAux* __restrict__ aux,
-                                                         WidePart* __restrict__ part,
-                                                         int y_is_f32) {
-    __shared__ double red[NT / kWave];
-    __shared__ int last;
-    const int c = wide[blockIdx.y];
-    const CurveGeom G = geom[c];
+// it also clears the record's counters for the kernels that follow.
+template <int KIND, bool F32, bool META>
+__global__ __launch_bounds__(kWideNT) void wide_reduce_kernel(MetaIn<META>, char* ws, int meta_words,
+                                                              int off_geom, int off_wide,
+                                                              const double* __restrict__ t,
+                                                              const void* __restrict__ a,
+                                                              const void* __restrict__ b,
+                                                              WideAux* __restrict__ aux,
+                                                              WidePart* __restrict__ part,
+                                                              int y_is_f32) {
+    constexpr int W = kWideNT / kWave;
+    constexpr int NQ = F32 ? 8 : 6;
+    __shared__ double red[NQ * W];
+    const char* const desc = meta_base<META>(ws, meta_words, kWideNT);
+    const int c = ((const int32_t*)(desc + off_wide))[blockIdx.y];
+    const CurveGeom& G = ((const CurveGeom*)(desc + off_geom))[c];
     WideAux& X = aux[blockIdx.y];
-    WidePart* P = part + (int64_t)blockIdx.y * gridDim.x;
     const int tid = threadIdx.x;
-    WidePart v{};
-    v.tmin = INFINITY;
-    v.tmax = -INFINITY;
-    const int j1 = min(G.n_obs, (int)(blockIdx.x + 1) * kWideChunk);
-    for (int j = (int)blockIdx.x * kWideChunk + tid; j < j1; j += NT) {
-        PrepVals p = load_point<KIND>(t, a, b, G.obs + j, y_is_f32);
-        v.tmin = fmin(v.tmin, p.t);
-        v.tmax = fmax(v.tmax, p.t);
-        if (F32 && isfinite(p.t)) {
-            v.st += p.t;
-            v.ct += 1.0;
-        }
-        if (KIND == 0) {
-            if (isfinite(p.yv)) {
-                v.sy += p.yv;
-                v.cy += 1.0;
-            }
-            const double iw = 1.0 / (p.wv * p.wv);
-            v.sw += iw;
-            v.swy += p.yv * iw;
-        }
-    }
-    auto reduce = [&](WidePart& q) {
-        q.tmin = block_min<NT>(q.tmin, red);
-        q.tmax = block_max<NT>(q.tmax, red);
-        if (F32) {
-            q.st = block_sum<NT>(q.st, red);
-            q.ct = block_sum<NT>(q.ct, red);
-        }
-        if (KIND == 0) {
-            q.sy = block_sum<NT>(q.sy, red);
-            q.cy = block_sum<NT>(q.cy, red);
-            q.sw = block_sum<NT>(q.sw, red);
-            q.swy = block_sum<NT>(q.swy, red);
+    const int lane = tid & (kWave - 1), wv = tid / kWave;
+    const WideSpan sp(G.n_obs);
+    if (sp.j0 >= sp.j1) return;
+    const int64_t obs = G.obs;
+    PrepVals q[kWidePts];
+    auto load = [&](int base) {
+#pragma unroll
+        for (int u = 0; u < kWidePts; ++u) {
+            const int j = base + u * kWideNT + tid;
+            if (j < sp.j1) q[u] = load_point<KIND>(t, a, b, obs + j, y_is_f32);
         }
     };
-    reduce(v);
-    if (tid == 0) P[blockIdx.x] = v;
-    __threadfence();
-    __syncthreads();
-    if (tid == 0) last = (atomicAdd(&X.red_done, 1) == (int)gridDim.x - 1);
-    __syncthreads();
-    if (!last) return;   // block-uniform
-    __threadfence();
-    WidePart q{};
-    q.tmin = INFINITY;
-    q.tmax = -INFINITY;
-    for (int i = tid; i < (int)gridDim.x; i += NT) {
-        const double* s = &P[i].tmin;
-        q.tmin = fmin(q.tmin, agent_load(s + 0));
-        q.tmax = fmax(q.tmax, agent_load(s + 1));
-        q.st += agent_load(s + 2);
-        q.ct += agent_load(s + 3);
-        q.sy += agent_load(s + 4);
-        q.cy += agent_load(s + 5);
-        q.sw += agent_load(s + 6);
-        q.swy += agent_load(s + 7);
+    load(sp.j0);
+    const int nb = (1 << G.p2) / G.c1;
+    for (int i = (int)blockIdx.x * kWideNT + tid; i < 2 * nb; i += sp.chunks * kWideNT) {
+        X.hist[i] = 0;
+        X.taken[i] = 0;
     }
-    reduce(q);
-    if (tid == 0) {
-        CurveState st;
-        st.tref = q.tmin;
-        st.tspan = q.tmax - q.tmin;
-        st.tmean = F32 ? q.st / q.ct : 0.0;
-        st.klow = low_count(G, st.tspan);
+    if (blockIdx.x == 0)
+        for (int i = tid; i < kLowSlots / 2; i += kWideNT) X.low_done[i] = 0;
+    double v[NQ] = {INFINITY, INFINITY};
+    sp.each(load, [&](int, int u) {
+        const PrepVals& p = q[u];
+        v[0] = fmin(v[0], p.t);
+        v[1] = fmin(v[1], -p.t);
         if (KIND == 0) {
-            const double ymean = q.sy / q.cy;
-            X.ymean = ymean;
-            X.s0inv = 1.0 / q.sw;
-            st.ybar = q.swy / q.sw - ymean;
-            st.yy = 0.0;   // the scatter's last block writes it
-        } else {
-            X.ymean = 0.0;
-            X.s0inv = 1.0;
-            st.ybar = G.ybar_in;
-            st.yy = G.yy_in;
+            if (isfinite(p.yv)) {
+                v[2] += p.yv;
+                v[3] += 1.0;
+            }
+            const double iw = 1.0 / (p.wv * p.wv);
+            v[4] += iw;
+            v[5] += p.yv * iw;
         }
-        state[c] = st;
+        if constexpr (F32)
+            if (isfinite(p.t)) {
+                v[NQ - 2] += p.t;
+                v[NQ - 1] += 1.0;
+            }
+    }, true);
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+        if (KIND != 0 && i >= 2 && i < 6) continue;
+        v[i] = i < 2 ? wave_min(v[i]) : wave_sum(v[i]);
+    }
+    if (lane == 0) {
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) red[i * W + wv] = v[i];
+    }
+    __syncthreads();
+    if (wv != 0) return;
+    block_fold<NQ>(red, lane, v);
+    if (lane == 0) {
+        WidePart& P = part[(int64_t)blockIdx.y * gridDim.x + blockIdx.x];
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) P.v[i] = v[i];
     }
 }
 
-// Bucketing of the wide curves' points over many blocks: blockIdx.y picks the
-// curve (wide[blockIdx.y], record aux[blockIdx.y]), blockIdx.x its chunk of
-// kWideChunk points.  Each block counts its chunk in LDS and adds the
-// non-zero counts to the record with one global atomic per bucket (per-point
-// global atomics on a few hundred counters serialise on their cache lines).
-// Counting: the last block of the curve to finish (the block count is
-// gridDim.x for every curve) scans the totals into the bucket starts bkt and
-// the cursors.  Scatter: each block reserves its slots per bucket with one
-// atomic on the cursor, then ranks its points in LDS.
-template <int KIND, bool F32>
-__device__ __forceinline__ void wide_chunk_counts(int (&h)[2][kMaxBuckets], const CurveGeom& G,
-                                                  const double* __restrict__ t, double tref,
+// this chunk's points per bucket of both node sets, h[0 .. NG nb)
+template <int KIND, bool F32, class Load, class Q>
+__device__ __forceinline__ void wide_chunk_counts(int* h, const CurveGeom& G, const WideSpan& sp,
+                                                  Load&& load, const Q& q, double tref,
                                                   double tmean, int m) {
     constexpr int NG = (KIND == 2) ? 1 : 2;
-    const int tid = threadIdx.x;
     const int n2 = 1 << G.p2;
-    const int nb = n2 / G.c1;
-    for (int i = tid; i < nb; i += NT) {
-        h[0][i] = 0;
-        h[1][i] = 0;
-    }
+    const int lc1 = 31 - __clz(G.c1);
+    const int nb = n2 >> lc1;
+    for (int i = threadIdx.x; i < NG * nb; i += kWideNT) h[i] = 0;
     __syncthreads();
-    const int j1 = min(G.n_obs, (int)(blockIdx.x + 1) * kWideChunk);
-    for (int j = (int)blockIdx.x * kWideChunk + tid; j < j1; j += NT) {
-        const double dt = point_dt<F32>(t[G.obs + j], tref, tmean);
-        if (!isfinite(dt)) continue;
+    sp.each(load, [&](int, int u) {
+        const double dt = point_dt<F32>(q[u].t, tref, tmean);
+        if (!isfinite(dt)) return;
 #pragma unroll
         for (int g = 1; g <= NG; ++g) {
             double yc;
             const int U = prep_cell<F32>(dt, g, G, m, yc);
-            atomicAdd(&h[g - 1][(U & (n2 - 1)) / G.c1], 1);
+            atomicAdd(&h[(g - 1) * nb + ((U & (n2 - 1)) >> lc1)], 1);
         }
-    }
+    }, true);
     __syncthreads();
 }
 
+// wide_count_kernel: every block folds the chunk partials, in chunk order (the
+// first writes the curve's state and weight constants), counts its chunk's
+// points per bucket in LDS and adds them to the record, two buckets in one 64-bit
+// atomic (no count reaches 2^32; per-point global atomics on a few hundred
+// counters would serialise on their cache lines).  It also sums its points'
+// (y - ymean - ybar)^2 / dy^2 (raw input).
 template <int KIND, bool F32>
-__global__ __launch_bounds__(NT) void wide_count_kernel(const CurveGeom* __restrict__ geom,
-                                                        const int32_t* __restrict__ wide,
-                                                        const CurveState* __restrict__ state,
-                                                        const double* __restrict__ t,
-                                                        WideAux* __restrict__ aux,
-                                                        int32_t* __restrict__ bkt, int m) {
-    __shared__ int h[2][kMaxBuckets];
-    __shared__ int wsum[NT / kWave + 1];
-    __shared__ int last;
+__global__ __launch_bounds__(kWideNT) void wide_count_kernel(const CurveGeom* __restrict__ geom,
+                                                             const int32_t* __restrict__ wide,
+                                                             CurveState* __restrict__ state,
+                                                             const double* __restrict__ t,
+                                                             const void* __restrict__ a,
+                                                             const void* __restrict__ b,
+                                                             WideAux* __restrict__ aux,
+                                                             WidePart* __restrict__ part, int m,
+                                                             int y_is_f32) {
+    constexpr int W = kWideNT / kWave;
+    constexpr int NQ = F32 ? 8 : 6;
     constexpr int NG = (KIND == 2) ? 1 : 2;
+    __shared__ double red[NQ * W];
+    __shared__ double redyy[W];
+    extern __shared__ __align__(16) int h[];
     const int tid = threadIdx.x;
-    const CurveGeom G = geom[wide[blockIdx.y]];
+    const int lane = tid & (kWave - 1), wv = tid / kWave;
+    const int c = wide[blockIdx.y];
+    const CurveGeom G = geom[c];
+    const WideSpan sp(G.n_obs);
+    if (sp.j0 >= sp.j1) return;
     WideAux& X = aux[blockIdx.y];
-    const int nb = (1 << G.p2) / G.c1;
-    const CurveState st = state[wide[blockIdx.y]];
-    wide_chunk_counts<KIND, F32>(h, G, t, st.tref, st.tmean, m);
+    PrepVals q[kWidePts];
+    auto load = [&](int base) {
 #pragma unroll
-    for (int g = 0; g < NG; ++g)
-        for (int i = tid; i < nb; i += NT)
-            if (h[g][i] != 0) atomicAdd(&X.hist[g][i], h[g][i]);
-    __threadfence();
-    __syncthreads();
-    if (tid == 0) last = (atomicAdd(&X.done, 1) == (int)gridDim.x - 1);
-    __syncthreads();
-    if (!last) return;   // block-uniform
-    __threadfence();
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-        for (int i = tid; i < nb; i += NT)
-            h[g][i] = __hip_atomic_load(&X.hist[g][i], __ATOMIC_RELAXED,
-                                        __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-        const int total = block_exclusive_scan<NT>(h[g], nb, wsum);
-        int32_t* bk = bkt + G.bkt + (int64_t)g * (nb + 1);
-        for (int i = tid; i < nb; i += NT) {
-            bk[i] = h[g][i];
-            X.hist[g][i] = h[g][i];
+        for (int u = 0; u < kWidePts; ++u) {
+            const int j = base + u * kWideNT + tid;
+            if (j < sp.j1) q[u] = load_point<KIND>(t, a, b, G.obs + j, y_is_f32);
         }
-        if (tid == 0) bk[nb] = total;
-        __syncthreads();
+    };
+    load(sp.j0);
+    WidePart* const P = part + (int64_t)blockIdx.y * gridDim.x;
+    double v[NQ] = {INFINITY, INFINITY};
+    for (int i = tid; i < sp.chunks; i += kWideNT) {
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) v[k] = k < 2 ? fmin(v[k], P[i].v[k]) : v[k] + P[i].v[k];
     }
-}
-
-// The scatter also sums (y - ymean - ybar)^2 / dy^2 per chunk (raw input);
-// its last block combines the chunks in order into the curve's yy.
-template <int KIND, bool F32>
-__global__ __launch_bounds__(NT) void wide_scatter_kernel(const CurveGeom* __restrict__ geom,
-                                                          const int32_t* __restrict__ wide,
-                                                          CurveState* __restrict__ state,
-                                                          const double* __restrict__ t,
-                                                          const void* __restrict__ a,
-                                                          const void* __restrict__ b,
-                                                          PointArrays pa,
-                                                          WideAux* __restrict__ aux,
-                                                          WidePart* __restrict__ part, int m,
-                                                          int y_is_f32) {
-    __shared__ int h[2][kMaxBuckets];
-    __shared__ double red[NT / kWave];
-    __shared__ int last;
-    constexpr int NG = (KIND == 2) ? 1 : 2;
-    const int tid = threadIdx.x;
-    const CurveGeom G = geom[wide[blockIdx.y]];
-    WideAux& X = aux[blockIdx.y];
-    const CurveState st = state[wide[blockIdx.y]];
-    const int nb = (1 << G.p2) / G.c1;
-    wide_chunk_counts<KIND, F32>(h, G, t, st.tref, st.tmean, m);
-    // this block's first slot in each bucket
 #pragma unroll
-    for (int g = 0; g < NG; ++g)
-        for (int i = tid; i < nb; i += NT)
-            if (h[g][i] != 0) h[g][i] = atomicAdd(&X.hist[g][i], h[g][i]);
+    for (int i = 0; i < NQ; ++i) {
+        if (KIND != 0 && i >= 2 && i < 6) continue;
+        v[i] = i < 2 ? wave_min(v[i]) : wave_sum(v[i]);
+    }
+    if (lane == 0) {
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) red[i * W + wv] = v[i];
+    }
     __syncthreads();
-    const double ymean = X.ymean, s0inv = X.s0inv;
-    const double Fc = G.f0 + (double)G.kc * G.df;
-    const int j1 = min(G.n_obs, (int)(blockIdx.x + 1) * kWideChunk);
-    double syy = 0.0;
-    for (int j = (int)blockIdx.x * kWideChunk + tid; j < j1; j += NT) {
-        PrepVals p = load_point<KIND>(t, a, b, G.obs + j, y_is_f32);
-        double w, yw;
-        prep_weights<KIND>(p, ymean, st.ybar, s0inv, w, yw);
-        if (KIND == 0) {
-            const double d = p.yv - ymean - st.ybar;
-            syy += d * d / (p.wv * p.wv);
-        }
-        prep_emit<KIND, F32>(pa, G, j, point_dt<F32>(p.t, st.tref, st.tmean), w, yw, Fc, m,
-                             [&](int gs, int bucket) { return atomicAdd(&h[gs][bucket], 1); });
+    block_fold<NQ>(red, lane, v);
+    const double tref = v[0], tmean = F32 ? v[NQ - 2] / v[NQ - 1] : 0.0;
+    double ymean = 0.0, ybar = G.ybar_in, s0inv = 1.0;
+    if (KIND == 0) {
+        ymean = v[2] / v[3];
+        s0inv = 1.0 / v[4];
+        ybar = v[5] / v[4] - ymean;
+    }
+    if (blockIdx.x == 0 && tid == 0) {
+        CurveState st;
+        st.tref = tref;
+        st.tspan = -v[1] - tref;
+        st.tmean = tmean;
+        st.klow = low_count(G, st.tspan);
+        st.ybar = ybar;
+        st.yy = G.yy_in;   // (raw input: the scatter's first block writes it)
+        X.ymean = ymean;
+        X.s0inv = s0inv;
+        state[c] = st;
+    }
+    wide_chunk_counts<KIND, F32>(h, G, sp, load, q, tref, tmean, m);
+    const int nb = (1 << G.p2) / G.c1;
+    for (int i = tid; i < NG * nb / 2; i += kWideNT) {
+        const unsigned long long two = ((const unsigned long long*)h)[i];
+        if (two != 0) atomicAdd((unsigned long long*)X.hist + i, two);
     }
     if (KIND != 0) return;
-    WidePart* P = part + (int64_t)blockIdx.y * gridDim.x;
-    syy = block_sum<NT>(syy, red);
-    if (tid == 0) P[blockIdx.x].syy = syy;
-    __threadfence();
+    double s2 = 0.0;
+    sp.each(load, [&](int, int u) {
+        const PrepVals& p = q[u];
+        const double d = p.yv - ymean - ybar;
+        s2 += d * d / (p.wv * p.wv);
+    }, true);
+    s2 = block_sum<kWideNT>(s2, redyy);
+    if (tid == 0) P[blockIdx.x].syy = s2;
+}
+
+// wide_scatter_kernel: each block scans the buckets' totals into their starts
+// (the first writes them to bkt and folds the chunks' variance partials, in
+// order, into the curve's yy), counts its chunk again, reserves its slots per
+// bucket with one atomic for two buckets, then ranks its points in LDS.
+template <int KIND, bool F32>
+__global__ __launch_bounds__(kWideNT) void wide_scatter_kernel(const CurveGeom* __restrict__ geom,
+                                                               const int32_t* __restrict__ wide,
+                                                               CurveState* __restrict__ state,
+                                                               const double* __restrict__ t,
+                                                               const void* __restrict__ a,
+                                                               const void* __restrict__ b,
+                                                               PointArrays pa,
+                                                               int32_t* __restrict__ bkt,
+                                                               WideAux* __restrict__ aux,
+                                                               const WidePart* __restrict__ part,
+                                                               int m, int y_is_f32) {
+    constexpr int W = kWideNT / kWave;
+    constexpr int NG = (KIND == 2) ? 1 : 2;
+    __shared__ double red[W];
+    __shared__ int wsum[W];
+    extern __shared__ __align__(16) int h[];   // counts, then the buckets' starts
+    const int tid = threadIdx.x;
+    const int c = wide[blockIdx.y];
+    const CurveGeom G = geom[c];
+    const WideSpan sp(G.n_obs);
+    if (sp.j0 >= sp.j1) return;
+    WideAux& X = aux[blockIdx.y];
+    PrepVals q[kWidePts];
+    auto load = [&](int base) {
+#pragma unroll
+        for (int u = 0; u < kWidePts; ++u) {
+            const int j = base + u * kWideNT + tid;
+            if (j < sp.j1) q[u] = load_point<KIND>(t, a, b, G.obs + j, y_is_f32);
+        }
+    };
+    load(sp.j0);
+    const double tref = state[c].tref, tmean = F32 ? state[c].tmean : 0.0, ybar = state[c].ybar;
+    const double ymean = X.ymean, s0inv = X.s0inv;
+    const int nb = (1 << G.p2) / G.c1;
+    int* const start = h + NG * nb;
+    for (int i = tid; i < NG * nb; i += kWideNT) start[i] = X.hist[i];
     __syncthreads();
-    if (tid == 0) last = (atomicAdd(&X.yy_done, 1) == (int)gridDim.x - 1);
+    // (both sets hold the same points: the second's starts begin at half the total)
+    const int total = block_exclusive_scan<kWideNT>(start, NG * nb, wsum) / NG;
+    if (blockIdx.x == 0) {
+        int32_t* const bk = bkt + G.bkt;
+        for (int i = tid; i < NG * nb; i += kWideNT) {
+            const int second = i >= nb ? 1 : 0;
+            bk[i + second] = start[i] - second * total;
+        }
+        if (tid < NG) bk[tid * (nb + 1) + nb] = total;
+        if (KIND == 0) {
+            const WidePart* const P = part + (int64_t)blockIdx.y * gridDim.x;
+            double s2 = 0.0;
+            for (int i = tid; i < sp.chunks; i += kWideNT) s2 += P[i].syy;
+            s2 = block_sum<kWideNT>(s2, red);
+            if (tid == 0) state[c].yy = s2 * s0inv;
+        }
+    }
+    wide_chunk_counts<KIND, F32>(h, G, sp, load, q, tref, tmean, m);
+    // this block's first slot in each bucket
+    for (int i = tid; i < NG * nb / 2; i += kWideNT) {
+        const unsigned long long two = ((const unsigned long long*)h)[i];
+        if (two == 0) continue;
+        const unsigned long long was = atomicAdd((unsigned long long*)X.taken + i, two);
+        const int off = 2 * i >= nb ? total : 0;   // (nb is even)
+        h[2 * i] = start[2 * i] + (int)(uint32_t)was - off;
+        h[2 * i + 1] = start[2 * i + 1] + (int)(uint32_t)(was >> 32) - off;
+    }
     __syncthreads();
-    if (!last) return;   // block-uniform
-    __threadfence();
-    double acc = 0.0;
-    for (int i = tid; i < (int)gridDim.x; i += NT) acc += agent_load(&P[i].syy);
-    acc = block_sum<NT>(acc, red);
-    if (tid == 0) state[wide[blockIdx.y]].yy = acc * s0inv;
+    const double Fc = G.f0 + (double)G.kc * G.df;
+    sp.each(load, [&](int j, int u) {
+        const PrepVals& p = q[u];
+        double w, yw;
+        prep_weights<KIND>(p, ymean, ybar, s0inv, w, yw);
+        prep_emit<KIND, F32>(pa, G, j, point_dt<F32>(p.t, tref, tmean), w, yw, Fc, m,
+                             [&](int gs, int bucket) { return atomicAdd(&h[gs * nb + bucket], 1); });
+    }, true);
 }
 
 }  // namespace
@@ -717,22 +760,19 @@ hipError_t launch_prep_t(const CurveGeom* d_geom, const int32_t* small, int nsma
 #undef GLS_PREP_LAUNCH
     if (nwide <= 0 || !split) return hipSuccess;
     const int off_wide = (int)((const char*)wide - ws);
-    if (meta && nblocks == 0)
-        hipLaunchKernelGGL((wide_clear_kernel<true>), dim3(nwide), dim3(NT), 0, s, in, ws,
-                           meta_words, off_geom, off_wide, aux);
-    else
-        hipLaunchKernelGGL((wide_clear_kernel<false>), dim3(nwide), dim3(NT), 0, s,
-                           MetaIn<false>{}, ws, meta_words, off_geom, off_wide, aux);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    const dim3 grid((unsigned)((wide_max_obs + kWideChunk - 1) / kWideChunk), (unsigned)nwide);
-#define GLS_WIDE_LAUNCH(K)                                                                    \
-    hipLaunchKernelGGL((wide_reduce_kernel<K, F32>), grid, dim3(NT), 0, s, d_geom, wide,       \
-                       state, t, a, b, aux, part, yf);                                        \
-    hipLaunchKernelGGL((wide_count_kernel<K, F32>), grid, dim3(NT), 0, s, d_geom, wide, state, \
-                       t, aux, bkt, pp.m);                                                    \
-    hipLaunchKernelGGL((wide_scatter_kernel<K, F32>), grid, dim3(NT), 0, s, d_geom, wide,      \
-                       state, t, a, b, pa, aux, part, pp.m, yf)
+    const dim3 grid((unsigned)std::min(kWideBlocks, (wide_max_obs + kWideChunk - 1) / kWideChunk),
+                    (unsigned)nwide);
+    const bool ride = meta && nblocks == 0;
+#define GLS_WIDE_REDUCE(K, M, IN)                                                             \
+    hipLaunchKernelGGL((wide_reduce_kernel<K, F32, M>), grid, dim3(kWideNT), 0, s, IN, ws,     \
+                       meta_words, off_geom, off_wide, t, a, b, aux, part, yf)
+#define GLS_WIDE_LAUNCH(K)                                                                     \
+    if (ride) GLS_WIDE_REDUCE(K, true, in);                                                    \
+    else GLS_WIDE_REDUCE(K, false, MetaIn<false>{});                                           \
+    hipLaunchKernelGGL((wide_count_kernel<K, F32>), grid, dim3(kWideNT), lds, s, d_geom, wide, \
+                       state, t, a, b, aux, part, pp.m, yf);                                   \
+    hipLaunchKernelGGL((wide_scatter_kernel<K, F32>), grid, dim3(kWideNT), 2 * lds, s, d_geom, \
+                       wide, state, t, a, b, pa, bkt, aux, part, pp.m, yf)
     if (kind == 0) {
         GLS_WIDE_LAUNCH(0);
     } else if (kind == 1) {
@@ -741,6 +781,7 @@ hipError_t launch_prep_t(const CurveGeom* d_geom, const int32_t* small, int nsma
         GLS_WIDE_LAUNCH(2);
     }
 #undef GLS_WIDE_LAUNCH
+#undef GLS_WIDE_REDUCE
     return hipGetLastError();
 }
 }  // namespace
