@@ -98,7 +98,7 @@ struct CurveGeom {
     int64_t grid;      // first float2 of this curve's grids (ngrids * grid_cells)
     double f0;
     double df;
-    double b;          // Gaussian width in cells^2
+    double n4inv;      // 4 / n: quarter turns per unit of the inter-pass twiddles
     double ybar_in;    // GLS_INPUT_WEIGHTED
     double yy_in;      // GLS_INPUT_WEIGHTED
     int32_t n_obs;

@@ -62,11 +62,15 @@ __global__ __launch_bounds__(pass1_threads(N1, C1)) void pass1_kernel(const Curv
     __shared__ signed char rexp[FIX ? N1 : 1];   // fixed-point exponent per row
     const int tid = threadIdx.x;
     const int n2 = 1 << p2;
-    const int nb = n2 / C1;
-    const int bid = xcd_logical_block(blockIdx.x, gridDim.x);
-    const int jb = bid % nb;
-    const int gi = (bid / nb) % ngrids;
-    const int ce = bid / (nb * ngrids);   // the curve's place in the bucket entry
+    // (1 or 3 grids and a power of two of tiles per grid: three divisions here
+    // took a tenth of a small tile's instructions, see the inter-pass twiddles)
+    const int lnb = p2 - ilog2_c(C1);
+    const int nb = 1 << lnb;
+    const unsigned bid = (unsigned)xcd_logical_block(blockIdx.x, gridDim.x);
+    const int jb = (int)(bid & (unsigned)(nb - 1));
+    const unsigned grid = bid >> lnb;
+    const int ce = (int)(ngrids == 3 ? grid / 3u : grid);   // the curve's place in the entry
+    const int gi = (int)grid - ngrids * ce;
     const CurveGeom& G = bgeom[ce];
     const int n = G.n;
     const int a = jb * C1;
@@ -109,13 +113,19 @@ __global__ __launch_bounds__(pass1_threads(N1, C1)) void pass1_kernel(const Curv
     for (int i = tid; i < TL / 2; i += NT1)
         reinterpret_cast<float4*>(tile)[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     build_twiddles<N1, NT1>(T, tid);
+    // Tiles of few points are bound by vector instructions (432 x 4: 96,000 tiles
+    // of 2,000 curves of 20 to 300 points), a sixth of them in these tables
+    // and the block's place above.  Quarter turns in FP64, as exact as the reduced
+    // ratio, and shifts there: 469 -> 431 us, the whole call 735 -> 713 us.
     for (int i = tid; i < C1 * (NH + 64); i += NT1) {
         const int jj = i / (NH + 64);
         const int r = i - jj * (NH + 64);
         const int u2 = a + jj;
         // u2 < 2^12, r < 64, r - 64 < 2^6: the products stay below 2^24
-        if (r < 64) elo[jj * 64 + r] = expi_ratio32((uint32_t)(u2 * r), n);
-        else ehi[jj * NH + (r - 64)] = expi_ratio32((uint32_t)(u2 * 64 * (r - 64)), n);
+        const uint32_t x = r < 64 ? (uint32_t)(u2 * r) : (uint32_t)(u2 * 64 * (r - 64));
+        // (the plain transforms keep the exact ratio: see expi_rev)
+        const float2 w = ngrids == 3 ? expi_turn4((double)x * G.n4inv) : expi_ratio32(x, n);
+        (r < 64 ? elo[jj * 64 + r] : ehi[jj * NH + (r - 64)]) = w;
     }
     __syncthreads();
 
@@ -261,7 +271,7 @@ hipError_t pass1_dispatch(bool fix, bool nts, const CurveGeom* bgeom, int ncurve
                           const PlanParams& pp, hipStream_t s) {
     constexpr int NT = pass1_threads(N1, C1);
     const int nb = (1 << p2) / C1;
-    if (nb < 1 || ngrids < 1) return hipErrorInvalidValue;
+    if (nb < 1 || (ngrids != 1 && ngrids != 3)) return hipErrorInvalidValue;
     const float ainv = 1.0f / ((float)pp.m + 0.5f);
     // curves per launch: blocks x threads within max_launch_items()
     const int64_t per_curve = (int64_t)ngrids * nb * NT;

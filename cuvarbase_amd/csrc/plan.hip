@@ -45,6 +45,7 @@ struct gls_plan {
     };
     std::vector<Bucket> buckets;   // one entry per chunk of a size bucket and spread mode
     int spread_mode = GLS_SPREAD_FLOAT;  // gls_params.spread
+    std::vector<double> width;           // per curve: Gaussian width in cells^2 (NFFT method)
     std::vector<int8_t> curve_fixed;     // per curve: pass 1 spreads it in fixed point
     std::vector<int> bucket_lane;  // 0: the caller's stream, j > 0: auxiliary stream j-1
     bool fork_buckets = false;     // run the lanes concurrently (gls_plan_set_fork)
@@ -263,6 +264,7 @@ int plan_nfft_geometry(gls_plan* P, int ngrids, Layout& L, int64_t total_pts,
     // (n1, p2, fixed-point spreading) -> curves
     std::map<std::tuple<int, int, int>, std::vector<int32_t>> by_size;
     P->curve_fixed.assign(P->ncurves, 0);
+    P->width.assign(P->ncurves, 0.0);
     int64_t bkt_ints = 0;
     for (int i = 0; i < P->ncurves; ++i) {
         CurveGeom& G = P->geom[i];
@@ -280,10 +282,12 @@ int plan_nfft_geometry(gls_plan* P, int ngrids, Layout& L, int64_t total_pts,
         G.p2 = p2;
         G.c1 = c1;
         G.kc = G.nf / 2;
-        G.b = gauss_b((double)n / (double)G.nf, m);
-        G.g_binv = (float)(1.4426950408889634 / G.b);
-        G.g_norm = (float)(1.0 / std::sqrt(M_PI * G.b));
-        G.g_bpi2 = (float)(G.b * M_PI * M_PI);
+        const double b = gauss_b((double)n / (double)G.nf, m);
+        P->width[i] = b;
+        G.n4inv = 4.0 / (double)n;
+        G.g_binv = (float)(1.4426950408889634 / b);
+        G.g_norm = (float)(1.0 / std::sqrt(M_PI * b));
+        G.g_bpi2 = (float)(b * M_PI * M_PI);
         G.ninv = 1.0f / (float)n;
         // GLS_SPREAD_AUTO: fixed point for curves of at least one point per
         // kFixedCellsPerPoint grid cells, where its integer adds outrun the
@@ -1008,7 +1012,7 @@ int gls_plan_curve_geometry(const gls_plan* plan, int32_t i, int64_t* n, int32_t
     if (n) *n = nfft ? (int64_t)G.n : 0;
     if (n1) *n1 = nfft ? G.n1 : 0;
     if (n2) *n2 = nfft ? (1 << G.p2) : 0;
-    if (b) *b = nfft ? G.b : 0.0;
+    if (b) *b = nfft ? plan->width[i] : 0.0;
     return GLS_OK;
 }
 
