@@ -188,6 +188,67 @@ __device__ __forceinline__ void dft_reg(float2 (&x)[R]) {
     }
 }
 
+// The same with input twiddles, x[r] <- sum_q x[q] w^q exp(+2 pi i q r / R), R a
+// power of two and 0 <= arg w < 2 pi / R: decimation in time, with w^(R/len)
+// exp(2 pi i j / len) as the twiddle of butterfly j at length len, so that the
+// powers of w need no products of their own.  A butterfly u +- t v takes six
+// multiply-adds: u + t v, and 2 u less that.  For R = 16 about 220 instructions,
+// against 290 of fourteen powers, fifteen products and dft_reg: 2,000 curves of 20
+// to 300 points at 20,000 frequencies 713 -> 688 us, 1,000 of 50 to 5,000 points
+// 4,326 -> 4,273 us, as tiles of few points are bound by vector instructions.
+//   Squares below 45 degrees are taken as 1 - 2 sin^2, without the rounding of
+// cos^2, which the later powers would multiply: RMS error of a transform of
+// normal deviates against 64 bits, powers by products and here: 4,096 elements
+// 4.5e-7 and 2.7e-7, 256 2.1e-7 and 1.3e-7, 64 as 8 x 8 1.2e-7 and 1.1e-7.  Radix
+// 4 has no power to gain by, and takes u - t v as it stands: 64 as 16 x 4 9.4e-8
+// and 9.1e-8.
+template <int R>
+__device__ __forceinline__ void dft_twiddled(float2 (&x)[R], float2 w) {
+    constexpr int LOG = ilog2_c(R);
+    constexpr RootsOfUnity<16> W{};
+    float2 y[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) y[brev_c(i, LOG)] = x[i];
+    float2 pw[LOG];   // w^(2^k)
+    pw[0] = w;
+#pragma unroll
+    for (int k = 1; k < LOG; ++k)
+        pw[k] = make_float2(k < LOG - 1 ? fmaf(-2.f * pw[k - 1].y, pw[k - 1].y, 1.f)
+                                        : pw[k - 1].x * pw[k - 1].x - pw[k - 1].y * pw[k - 1].y,
+                            2.f * pw[k - 1].x * pw[k - 1].y);
+#pragma unroll
+    for (int lev = 1; lev <= LOG; ++lev) {
+        const int len = 1 << lev, half = len >> 1;
+        const int nt = len >= 4 ? len / 4 : 1;   // distinct twiddles up to a factor i
+        float2 t[R >= 4 ? R / 4 : 1];
+#pragma unroll
+        for (int j = 0; j < nt; ++j) {
+            const int e = j * (16 / len);
+            t[j] = j == 0 ? pw[LOG - lev] : cmul(pw[LOG - lev], make_float2(W.c[e], W.s[e]));
+        }
+#pragma unroll
+        for (int i = 0; i < R; i += len) {
+#pragma unroll
+            for (int j = 0; j < half; ++j) {
+                const float2 u = y[i + j], v = y[i + j + half];
+                const float2 a = t[j % nt];
+                const float2 b = j < nt ? a : make_float2(-a.y, a.x);   // times i
+                float2 p = make_float2(fmaf(b.x, v.x, u.x), fmaf(b.x, v.y, u.y));
+                p = make_float2(fmaf(-b.y, v.y, p.x), fmaf(b.y, v.x, p.y));
+                y[i + j] = p;
+                if (R == 4) {
+                    const float2 q = make_float2(fmaf(-b.x, v.x, u.x), fmaf(-b.x, v.y, u.y));
+                    y[i + j + half] = make_float2(fmaf(b.y, v.y, q.x), fmaf(-b.y, v.x, q.y));
+                } else {
+                    y[i + j + half] = make_float2(fmaf(2.f, u.x, -p.x), fmaf(2.f, u.y, -p.y));
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i) x[i] = y[i];
+}
+
 // exp(2 pi i q / n) for 0 <= q < 2^31 and 0 < n <= 2^24, evaluated from the
 // exactly reduced ratio (|2q'| <= n is exact in FP32) with a 32-bit remainder
 __device__ __forceinline__ float2 expi_ratio32(uint32_t q, uint32_t n) {
@@ -280,7 +341,8 @@ struct LdsRun {
 // Butterfly beta (b = beta % B, j = beta / B) reads x[j + q L/R], multiplies
 // input q by w^q, w = exp(2 pi i k / (NS R)), k = j % NS, and its output q
 // goes to index (j - k) R + k + q NS.
-template <int L, int B, int BS, int R, int NS, int NT>
+// FUSED: powers of two take their twiddles inside the butterflies (dft_twiddled)
+template <int L, int B, int BS, int R, int NS, int NT, bool FUSED>
 struct StockhamStage {
     static constexpr int LR = L / R;
     static constexpr int NBUT = LR * B;               // butterflies in the stage
@@ -304,7 +366,10 @@ struct StockhamStage {
 #pragma unroll
                     for (int q = 0; q < R; ++q) x[r][q] = s[run.at(q)];
                 }
-                if constexpr (NS > 1) {
+                if constexpr (NS > 1 && FUSED && (R & (R - 1)) == 0) {
+                    dft_twiddled<R>(x[r], tw_lookup<L>(T, j % NS * (L / (NS * R))));
+                    continue;
+                } else if constexpr (NS > 1) {
                     const int k = j % NS;
                     float2 w[R];
                     w[1] = tw_lookup<L>(T, k * (L / (NS * R)));
@@ -386,13 +451,13 @@ struct StockhamStage {
     }
 };
 
-template <int L, int B, int BS, int NS, int NT>
+template <int L, int B, int BS, int NS, int NT, bool FUSED>
 struct LdsFftStages {
     static __device__ __forceinline__ void run(float2* s, const TwTable<L>& T, int tid) {
         if constexpr (NS < L) {
             constexpr int R = next_radix(L / NS);
-            StockhamStage<L, B, BS, R, NS, NT>::run(s, T, tid);
-            LdsFftStages<L, B, BS, NS * R, NT>::run(s, T, tid);
+            StockhamStage<L, B, BS, R, NS, NT, FUSED>::run(s, T, tid);
+            LdsFftStages<L, B, BS, NS * R, NT, FUSED>::run(s, T, tid);
         }
     }
     // all stages in place except the last, whose outputs go to
@@ -402,10 +467,10 @@ struct LdsFftStages {
     static __device__ __forceinline__ void run_to(float2* s, const TwTable<L>& T, int tid,
                                                   F&& sink) {
         constexpr int R = next_radix(L / NS);
-        using St = StockhamStage<L, B, BS, R, NS, NT>;
+        using St = StockhamStage<L, B, BS, R, NS, NT, FUSED>;
         if constexpr (NS * R < L) {
             St::run(s, T, tid);
-            LdsFftStages<L, B, BS, NS * R, NT>::run_to(s, T, tid, sink);
+            LdsFftStages<L, B, BS, NS * R, NT, FUSED>::run_to(s, T, tid, sink);
         } else {
             float2 x[St::NB][R];
             St::compute(s, T, tid, x);
@@ -414,41 +479,32 @@ struct LdsFftStages {
     }
 };
 
-// Full in-place FFT (natural order in and out) of B sequences of length L
-// stored at s[lds_at<BS>(i, b)].  The caller has synchronised after writing s and T;
-// returns synchronised.
-template <int L, int B, int BS, int NT>
-__device__ __forceinline__ void lds_fft(float2* s, const TwTable<L>& T, int tid) {
-    static_assert(L >= 2 && L <= 4096 && smooth235(L), "L must be 2^a 3^b 5^c <= 4096");
-    LdsFftStages<L, B, BS, 1, NT>::run(s, T, tid);
-}
-
-// The same transform with the first stage's inputs read from src(j, q, LR, b)
-// (element j + q LR of sequence b, LR = L / first radix)
-// (natural order index i of sequence b) rather than from s: the loads of all
-// of a thread's first-stage butterflies are in flight together.  s need not
-// be initialised; T must be complete at the first barrier.  Returns
-// synchronised with the result in s.
-template <int L, int B, int BS, int NT, class S>
+// FFT (natural order in and out) of B sequences of length L at s[lds_at<BS>(i,
+// b)], with the first stage's inputs read from src(j, q, LR, b) (element j + q LR
+// of sequence b, LR = L / first radix) rather than from s: the loads of all of a
+// thread's first-stage butterflies are in flight together.  s need not be
+// initialised; T must be complete at the first barrier.  Returns synchronised
+// with the result in s.
+template <int L, int B, int BS, int NT, bool FUSED, class S>
 __device__ __forceinline__ void lds_fft_from(float2* s, const TwTable<L>& T, int tid, S&& src) {
     static_assert(L >= 2 && L <= 4096 && smooth235(L), "L must be 2^a 3^b 5^c <= 4096");
     constexpr int R = next_radix(L);
-    using St = StockhamStage<L, B, BS, R, 1, NT>;
+    using St = StockhamStage<L, B, BS, R, 1, NT, FUSED>;
     float2 x[St::NB][R];
     St::compute_from(src, tid, x);
     St::emit_lds(s, tid, x);
     __syncthreads();
-    LdsFftStages<L, B, BS, R, NT>::run(s, T, tid);
+    LdsFftStages<L, B, BS, R, NT, FUSED>::run(s, T, tid);
 }
 
-// The same transform with the last stage's outputs handed to
-// sink(base, q, NS, b, v) (index base + q NS of sequence b)
-// (natural order index i of sequence b) instead of being stored; s is left
-// holding the second-to-last stage.  No barrier at the end.
-template <int L, int B, int BS, int NT, class F>
+// The same transform of sequences in s (the caller has synchronised after
+// writing s and T), with the last stage's outputs handed to sink(base, q, NS, b,
+// v) (index base + q NS of sequence b) instead of being stored; s is left holding
+// the second-to-last stage.  No barrier at the end.
+template <int L, int B, int BS, int NT, bool FUSED, class F>
 __device__ __forceinline__ void lds_fft_to(float2* s, const TwTable<L>& T, int tid, F&& sink) {
     static_assert(L >= 2 && L <= 4096 && smooth235(L), "L must be 2^a 3^b 5^c <= 4096");
-    LdsFftStages<L, B, BS, 1, NT>::run_to(s, T, tid, sink);
+    LdsFftStages<L, B, BS, 1, NT, FUSED>::run_to(s, T, tid, sink);
 }
 
 // LDS row stride for B interleaved sequences (bank spreading comes from the

@@ -43,9 +43,11 @@ constexpr int pass1_threads(int n1, int c1) { return n1 * c1 >= 6144 ? 512 : 256
 // C1: grid columns per workgroup (one LDS tile of N1 x C1 cells)
 // NTS: the grids are stored non-temporally (launches whose grids are larger
 // than the memory-side cache; pass 2 reads them from HBM either way)
-template <int N1, int C1, bool FIX, bool NTS>
+// NG: the three grids of a curve, or one of a plain transform, which keeps the
+// twiddles' separate products and exact ratios: see expi_rev
+template <int N1, int C1, int NG, bool FIX, bool NTS>
 __global__ __launch_bounds__(pass1_threads(N1, C1)) void pass1_kernel(const CurveGeom* __restrict__ bgeom,
-                                                    int ngrids, int p2, PointArrays pa,
+                                                    int p2, PointArrays pa,
                                                     const int32_t* __restrict__ bkt,
                                                     float2* __restrict__ grids, int m,
                                                     int window, float es_beta, float ainv) {
@@ -62,15 +64,15 @@ __global__ __launch_bounds__(pass1_threads(N1, C1)) void pass1_kernel(const Curv
     __shared__ signed char rexp[FIX ? N1 : 1];   // fixed-point exponent per row
     const int tid = threadIdx.x;
     const int n2 = 1 << p2;
-    // (1 or 3 grids and a power of two of tiles per grid: three divisions here
-    // took a tenth of a small tile's instructions, see the inter-pass twiddles)
+    // (a known number of grids and a power of two of tiles per grid: three divisions
+    // here took a tenth of a small tile's instructions, see the inter-pass twiddles)
     const int lnb = p2 - ilog2_c(C1);
     const int nb = 1 << lnb;
     const unsigned bid = (unsigned)xcd_logical_block(blockIdx.x, gridDim.x);
     const int jb = (int)(bid & (unsigned)(nb - 1));
     const unsigned grid = bid >> lnb;
-    const int ce = (int)(ngrids == 3 ? grid / 3u : grid);   // the curve's place in the entry
-    const int gi = (int)grid - ngrids * ce;
+    const int ce = (int)(grid / (unsigned)NG);   // the curve's place in the bucket entry
+    const int gi = (int)grid - NG * ce;
     const CurveGeom& G = bgeom[ce];
     const int n = G.n;
     const int a = jb * C1;
@@ -123,8 +125,7 @@ __global__ __launch_bounds__(pass1_threads(N1, C1)) void pass1_kernel(const Curv
         const int u2 = a + jj;
         // u2 < 2^12, r < 64, r - 64 < 2^6: the products stay below 2^24
         const uint32_t x = r < 64 ? (uint32_t)(u2 * r) : (uint32_t)(u2 * 64 * (r - 64));
-        // (the plain transforms keep the exact ratio: see expi_rev)
-        const float2 w = ngrids == 3 ? expi_turn4((double)x * G.n4inv) : expi_ratio32(x, n);
+        const float2 w = NG == 3 ? expi_turn4((double)x * G.n4inv) : expi_ratio32(x, n);
         (r < 64 ? elo[jj * 64 + r] : ehi[jj * NH + (r - 64)]) = w;
     }
     __syncthreads();
@@ -240,7 +241,7 @@ __global__ __launch_bounds__(pass1_threads(N1, C1)) void pass1_kernel(const Curv
     // (elo[0] = 1 exactly, so the product needs no special case; when the
     // output stride ns is a multiple of 64 a butterfly's outputs share one elo
     // entry and step through ehi, and the stride goes to the scalar offset)
-    lds_fft_to<N1, C1, BS, NT1>(tile, T, tid, [&](int kb, int q, int ns, int jj, float2 v) {
+    lds_fft_to<N1, C1, BS, NT1, NG == 3>(tile, T, tid, [&](int kb, int q, int ns, int jj, float2 v) {
         float2 w;
         if ((ns & 63) == 0) {
             w = cmul(ehi[jj * NH + (kb >> 6) + q * (ns >> 6)], elo[jj * 64 + (kb & 63)]);
@@ -281,15 +282,19 @@ hipError_t pass1_dispatch(bool fix, bool nts, const CurveGeom* bgeom, int ncurve
         const dim3 grid((unsigned)((int64_t)cnt * ngrids * nb));
         // a curve's bucket offsets follow its predecessors', 2 (nb + 1) each
         const int32_t* bk = bkt + (int64_t)c0 * 2 * (nb + 1);
-#define GLS_P1_LAUNCH(F, S)                                                                    \
-    hipLaunchKernelGGL((pass1_kernel<N1, C1, F, S>), grid, dim3(NT), 0, s, bgeom + c0, ngrids, \
-                       p2, pa, bk, grids, pp.m, pp.window, pp.es_beta, ainv)
-        if (fix) {
-            if (nts) GLS_P1_LAUNCH(true, true);
-            else GLS_P1_LAUNCH(true, false);
+#define GLS_P1_LAUNCH(G, F, S)                                                                    \
+    hipLaunchKernelGGL((pass1_kernel<N1, C1, G, F, S>), grid, dim3(NT), 0, s, bgeom + c0, p2, pa, \
+                       bk, grids, pp.m, pp.window, pp.es_beta, ainv)
+        if (ngrids == 1) {   // (plans of plain transforms spread with FP32 atomics)
+            if (fix) return hipErrorInvalidValue;
+            if (nts) GLS_P1_LAUNCH(1, false, true);
+            else GLS_P1_LAUNCH(1, false, false);
+        } else if (fix) {
+            if (nts) GLS_P1_LAUNCH(3, true, true);
+            else GLS_P1_LAUNCH(3, true, false);
         } else {
-            if (nts) GLS_P1_LAUNCH(false, true);
-            else GLS_P1_LAUNCH(false, false);
+            if (nts) GLS_P1_LAUNCH(3, false, true);
+            else GLS_P1_LAUNCH(3, false, false);
         }
 #undef GLS_P1_LAUNCH
         const hipError_t e = hipGetLastError();

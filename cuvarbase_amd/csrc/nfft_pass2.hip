@@ -50,7 +50,8 @@ __global__ __launch_bounds__(pass2_threads_for(P2, CR, OUT)) void pass2_kernel(
     const uint32_t gs = (uint32_t)grid_cells(n1, P2);   // cells of one grid
     const __amdgpu_buffer_rsrc_t src = grid_rsrc(grids + G.grid, 8u * (NG * gs));
     build_twiddles<N2, NT>(T, tid);
-    lds_fft_from<N2, B, BS, NT>(tile, T, tid, [&](int j, int q, int lr, int bb) -> float2 {
+    // (plain transforms keep the separate twiddle products: see expi_rev)
+    lds_fft_from<N2, B, BS, NT, OUT != 2>(tile, T, tid, [&](int j, int q, int lr, int bb) -> float2 {
         // column u2 = j + q lr of row `row` in the row-block layout.  Rows past
         // n1 (a partial last block) read row n1 - 1 instead; their transforms
         // are never emitted
