@@ -28,6 +28,29 @@ namespace {
 // columns of the long lengths), 256 below
 constexpr int pass1_threads(int n1, int c1) { return n1 * c1 >= 6144 ? 512 : 256; }
 
+// The inter-pass twiddles of a column's n1 rows are products of two tables, of the
+// rows 0 .. LO - 1 and of the multiples of LO.  LO is the power of two that costs
+// least: n1 / LO + LO entries of about 50 instructions, and about 4 per row if the
+// last stage's output stride is no multiple of LO (a butterfly's outputs then share
+// no entry, and their places are worked out one by one).  Against 64 throughout
+// (the plain transforms': they keep their roundings): 432 x 4, 43 entries a column
+// for 71, 440 -> 408 us for 96,000 tiles; 2160 x 1, where 53 more entries buy the
+// shared places, 132 -> 126 us; 1,000 curves of 50 to 5,000 points 5,190 -> 5,120
+// us of kernels.
+constexpr int twiddle_split(int n1) {
+    int last = n1;   // the last stage's radix
+    while (last != next_radix(last)) last /= next_radix(last);
+    int best = 64, least = 1 << 30;
+    for (int lo = 8; lo <= 64; lo *= 2) {
+        const int cost = (n1 + lo - 1) / lo + lo + ((n1 / last) % lo != 0 ? n1 / 12 : 0);
+        if (cost <= least) {
+            least = cost;
+            best = lo;
+        }
+    }
+    return best;
+}
+
 // ---------------------------------------------------------------------------
 // pass 1: spread + column FFT + inter-pass twiddle
 // ---------------------------------------------------------------------------
@@ -54,13 +77,14 @@ __global__ __launch_bounds__(pass1_threads(N1, C1)) void pass1_kernel(const Curv
     static_assert(pass1_tile_ok(N1, C1), "pass-1 tile out of range");
     constexpr int NT1 = pass1_threads(N1, C1);
     constexpr int BS = lds_stride(C1);
-    constexpr int NH = (N1 + 63) / 64;
+    constexpr int LO = NG == 3 ? twiddle_split(N1) : 64, LLO = ilog2_c(LO);
+    constexpr int NH = (N1 + LO - 1) / LO;
     // (rounded up to whole 16-byte pairs so that it is cleared with 128-bit stores)
     constexpr int TL = (lds_size(N1, BS) + 1) & ~1;
     __shared__ __align__(16) float2 tile[TL];
     __shared__ TwTable<N1> T;
-    __shared__ float2 ehi[C1 * NH];   // exp(2 pi i u2 64 kh / n)
-    __shared__ float2 elo[C1 * 64];   // exp(2 pi i u2 kl / n)
+    __shared__ float2 ehi[C1 * NH];   // exp(2 pi i u2 LO kh / n)
+    __shared__ float2 elo[C1 * LO];   // exp(2 pi i u2 kl / n)
     __shared__ signed char rexp[FIX ? N1 : 1];   // fixed-point exponent per row
     const int tid = threadIdx.x;
     const int n2 = 1 << p2;
@@ -119,14 +143,14 @@ __global__ __launch_bounds__(pass1_threads(N1, C1)) void pass1_kernel(const Curv
     // of 2,000 curves of 20 to 300 points), a sixth of them in these tables
     // and the block's place above.  Quarter turns in FP64, as exact as the reduced
     // ratio, and shifts there: 469 -> 431 us, the whole call 735 -> 713 us.
-    for (int i = tid; i < C1 * (NH + 64); i += NT1) {
-        const int jj = i / (NH + 64);
-        const int r = i - jj * (NH + 64);
+    for (int i = tid; i < C1 * (NH + LO); i += NT1) {
+        const int jj = i / (NH + LO);
+        const int r = i - jj * (NH + LO);
         const int u2 = a + jj;
-        // u2 < 2^12, r < 64, r - 64 < 2^6: the products stay below 2^24
-        const uint32_t x = r < 64 ? (uint32_t)(u2 * r) : (uint32_t)(u2 * 64 * (r - 64));
+        // u2 < 2^12, r and LO (r - LO) < n1 <= 2^12: the products stay below 2^24
+        const uint32_t x = r < LO ? (uint32_t)(u2 * r) : (uint32_t)(u2 * LO * (r - LO));
         const float2 w = NG == 3 ? expi_turn4((double)x * G.n4inv) : expi_ratio32(x, n);
-        (r < 64 ? elo[jj * 64 + r] : ehi[jj * NH + (r - 64)]) = w;
+        (r < LO ? elo[jj * LO + r] : ehi[jj * NH + (r - LO)]) = w;
     }
     __syncthreads();
 
@@ -239,15 +263,15 @@ __global__ __launch_bounds__(pass1_threads(N1, C1)) void pass1_kernel(const Curv
     const __amdgpu_buffer_rsrc_t out = grid_rsrc(grids + G.grid + gi * gs, 8u * (uint32_t)gs);
     const int rb = kRowBlock << p2;          // cells of one row block
     // (elo[0] = 1 exactly, so the product needs no special case; when the
-    // output stride ns is a multiple of 64 a butterfly's outputs share one elo
+    // output stride ns is a multiple of LO a butterfly's outputs share one elo
     // entry and step through ehi, and the stride goes to the scalar offset)
     lds_fft_to<N1, C1, BS, NT1, NG == 3>(tile, T, tid, [&](int kb, int q, int ns, int jj, float2 v) {
         float2 w;
-        if ((ns & 63) == 0) {
-            w = cmul(ehi[jj * NH + (kb >> 6) + q * (ns >> 6)], elo[jj * 64 + (kb & 63)]);
+        if ((ns & (LO - 1)) == 0) {
+            w = cmul(ehi[jj * NH + (kb >> LLO) + q * (ns >> LLO)], elo[jj * LO + (kb & (LO - 1))]);
         } else {
             const int k1 = kb + q * ns;
-            w = cmul(ehi[jj * NH + (k1 >> 6)], elo[jj * 64 + (k1 & 63)]);
+            w = cmul(ehi[jj * NH + (k1 >> LLO)], elo[jj * LO + (k1 & (LO - 1))]);
         }
         // row-block layout: when the output stride ns is a multiple of the
         // block height, a butterfly's outputs share their in-block offset and
