@@ -38,8 +38,7 @@ constexpr int pass1_threads(int n1, int c1) { return n1 * c1 >= 6144 ? 512 : 256
 // shared places, 132 -> 126 us; 1,000 curves of 50 to 5,000 points 5,190 -> 5,120
 // us of kernels.
 constexpr int twiddle_split(int n1) {
-    int last = n1;   // the last stage's radix
-    while (last != next_radix(last)) last /= next_radix(last);
+    const int last = last_radix(n1, true);
     int best = 64, least = 1 << 30;
     for (int lo = 8; lo <= 64; lo *= 2) {
         const int cost = (n1 + lo - 1) / lo + lo + ((n1 / last) % lo != 0 ? n1 / 12 : 0);

@@ -22,7 +22,8 @@ TOL = 5e-6
 @pytest.mark.parametrize("spread", [_lib.SPREAD_FLOAT, _lib.SPREAD_FIXED], ids=["float", "fixed"])
 @pytest.mark.parametrize("n1,p2", [(16, 12), (40, 11), (48, 10), (72, 9), (80, 8), (128, 7),
                                    (144, 6), (200, 9), (256, 8), (384, 7), (400, 6), (405, 6),
-                                   (432, 6), (640, 6), (768, 6), (1280, 6), (2048, 6), (2304, 6),
+                                   (432, 6), (640, 6), (648, 6), (768, 6), (1080, 6), (1152, 6),
+                                   (1280, 6), (2048, 6), (2160, 6), (2304, 6),
                                    (3072, 6), (3200, 6), (3240, 6), (3456, 6), (4096, 6)])
 def test_stages_against_direct_sums(n1, p2, spread):
     rng = np.random.default_rng(n1)
