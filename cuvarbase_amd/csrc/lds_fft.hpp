@@ -241,8 +241,8 @@ __device__ __forceinline__ void dft_reg(float2 (&x)[R]) {
 // powers of w need no products of their own.  A butterfly u +- t v takes six
 // multiply-adds: u + t v, and 2 u less that.  For R = 16 about 220 instructions,
 // against 290 of fourteen powers, fifteen products and dft_reg: 2,000 curves of 20
-// to 300 points at 20,000 frequencies 713 -> 688 us, 1,000 of 50 to 5,000 points
-// 4,326 -> 4,273 us, as tiles of few points are bound by vector instructions.
+// to 300 points at 20,000 frequencies 713 -> 700 us, 1,000 of 50 to 5,000 points
+// 4,326 -> 4,290 us, as tiles of few points are bound by vector instructions.
 //   Squares below 45 degrees are taken as 1 - 2 sin^2, without the rounding of
 // cos^2, which the later powers would multiply: RMS error of a transform of
 // normal deviates against 64 bits, powers by products and here: 4,096 elements

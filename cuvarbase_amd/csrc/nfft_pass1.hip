@@ -126,7 +126,7 @@ __global__ __launch_bounds__(pass1_threads(N1, C1)) void pass1_kernel(const Curv
     // A thread spreads a point's C1 taps in turn, or, in a tile of few points, C1
     // consecutive threads take a column each: 1 or 2 steps instead of C1, and lanes
     // that would have no point have a tap.  (432 x 4, mostly 20 to 100 points a tile:
-    // 408 -> 380 us for 96,000 tiles, 2,000 curves of 20 to 300 points 691 -> 662 us.
+    // 408 -> 376 us for 96,000 tiles, 2,000 curves of 20 to 300 points 691 -> 662 us.
     // With more points than PF rounds hold, whose records are all on their way at
     // once, a column per thread waits for each round's: 128 x 16 of some 1,500 points
     // 34 -> 49 us.)
